@@ -108,6 +108,12 @@ struct sgpu_timer_acc {
     int count = 0;
 };
 
+// How stencil_march covers a block (0 rows: it does not apply): gx 16-byte
+// groups per row, ty rows and zchunk planes per workgroup.
+struct sgpu_march_plan {
+    int gx = 0, ty = 0, zchunk = 0;
+};
+
 struct sgpu_context {
     int device = 0;
     int nx = 0, ny = 0, nz = 0;
@@ -125,10 +131,13 @@ struct sgpu_context {
     // on grids of 81-96 / 65-80 points), 13 / 14 = the same shapes as
     // stencil_rows when nx is exactly 96 / 80 (FP32); -1 (default) = the
     // fastest of 0 / 7 / 8 (9 / 10 below 16 columns, 11-14 where they fit),
-    // timed once per (precision, column count) and kept in tile_choice.  SPARC_AMD_STENCIL_TILE fixes one at
-    // creation.
+    // timed once per (precision, column count) and kept in tile_choice.  Above
+    // them, from 16 planes and 20 points along x: 20 = stencil_march, 21 =
+    // stencil_near, chosen by the block's bytes without timing.
+    // SPARC_AMD_STENCIL_TILE fixes one at creation.
     int stencil_cfg = -1;
     std::map<std::pair<int, int>, int> tile_choice;
+    std::map<std::pair<int, int>, sgpu_march_plan> march_plans;
     // fuse each filter step's nonlocal projection into the previous step's
     // apply (SPARC_AMD_NL_CHAIN=0 turns it off; results are bitwise equal)
     bool nl_chain = true;

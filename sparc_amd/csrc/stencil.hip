@@ -10,7 +10,12 @@
 // Periodic halos wrap indices (the reference copies the opposite face,
 // :536-577); Dirichlet halos read zero.
 //
-// Two kernels:
+// Kernels:
+//  * stencil_march<T, HV, HZ, PART>: radius 6, the default for blocks above
+//    3.6 MB: whole x-rows, 16 bytes per thread, a block of rows marching along z
+//    with the z sums pending in registers.
+//  * stencil_near<T, HV, HZ>: radius 6, the default for smaller blocks: every
+//    neighbour straight from L2.
 //  * stencil_tiled<T, TX, TY, RY>: radius 6.  A TX x TY tile of the x-y plane
 //    (plus a 6-deep halo) is staged in LDS per z-plane while the block marches
 //    along z; each thread keeps a 13-deep register queue of its own points'
@@ -564,6 +569,362 @@ __global__ __launch_bounds__(TX *(TY / RY)) void stencil_ring(StencilParams<T> p
     }
 }
 
+// Marching form for large blocks: radius 6, whole x-rows, 16 bytes (V points
+// of one row) per thread.  A block owns ty rows of one column and marches
+// along z; a plane is read once, interior and y halo together.  The plane's
+// x / y sums come from LDS (one buffer of whole rows with the x halo cells
+// filled from the row itself, double-buffered, one barrier per plane), and its
+// z contributions are added to the pending sums of the 12 output planes
+// around it: acc[k] is output plane p - 6 + k, and the shift by one plane is
+// free because every accumulator is rewritten as acc[k] = acc[k + 1] + w x.
+//
+// What bounds it: HBM, at 4.1 - 4.8 TB/s of x, z and out once each (a copy
+// reaches 4.7); with its loads returning zeros the 96^3 x 512 FP32 launch still
+// takes 0.66 of its 1.14 ms.  Per point 41 VALU operations and 64 bytes of LDS
+// reads (144 in FP64) against 60 and 96 (192) for stencil_tiled, whose scalar
+// LDS reads and 13-deep register queue (a move per plane and point) kept the
+// issue slots busy; and because the halo rows of a plane are read when the
+// neighbouring blocks read them as interior, they come from L2.  Recurrence
+// launch, stencil_tiled -> stencil_march: 96^3 x 512 FP32 1.36 -> 1.14 ms,
+// 78^3 x 480 FP32 840 -> 655 us, FP64 1.75 -> 1.22 ms, 52^3 x 160 FP32
+// 100 -> 61 us, FP64 211 -> 130 us, 128^3 x 1 FP64 20.4 -> 16.7 us.
+// A column as a raw buffer resource, the plane's offset in the scalar operand.
+// 16-byte accesses need the element's alignment only; dwords past the column
+// (the last row's last group, or kNoRow) read zero and are not stored.  Each
+// dword is range-checked by itself against offset + scalar offset, so partial
+// groups and absent rows need no branches.
+template <typename T>
+struct Column {
+    static constexpr int V = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    __amdgpu_buffer_rsrc_t r;
+    unsigned pb;
+    __device__ __forceinline__ Column(const T *base, int plane_bytes, int nz)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, plane_bytes * nz, 0x00020000)),
+          pb(plane_bytes)
+    {
+    }
+    __device__ __forceinline__ vec load(int plane, int off) const
+    {
+        return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(r, off, plane * pb, 0));
+    }
+    // Stores take the plane in the vector offset: the wait the compiler puts
+    // between a 16-byte store and the next write of its data registers is left
+    // out for a scalar offset, and without it that write reached the store
+    // (seen as wrong low words in FP64).  kNoRow + plane stays below 2^32.
+    __device__ __forceinline__ void store(int plane, int off, vec v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, off + plane * pb, 0, 0);
+    }
+    __device__ __forceinline__ T load1(int plane, int off) const
+    {
+        if constexpr (V == 4)
+            return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, plane * pb, 0));
+        else
+            return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, plane * pb, 0));
+    }
+    __device__ __forceinline__ void store1(int plane, int off, T v) const
+    {
+        if constexpr (V == 4)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off + plane * pb, 0, 0);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, off + plane * pb, 0, 0);
+    }
+    // the first rem (1 .. V - 1) values; off2 / off1: where the pair and the
+    // single value of them go (kNoRow: nowhere)
+    __device__ __forceinline__ void store_part(int plane, int off2, int off1, vec v, int rem) const
+    {
+        const u4 u = __builtin_bit_cast(u4, v);
+        __builtin_amdgcn_raw_buffer_store_b64(u2{u[0], u[1]}, r, off2 + plane * pb, 0, 0);
+        if constexpr (V == 4)
+            __builtin_amdgcn_raw_buffer_store_b32((rem & 2) ? u[2] : u[0], r, off1 + plane * pb, 0, 0);
+    }
+};
+constexpr int kNoRow = 0x7ffffff0;  // past every column
+
+// w x + a in a register of its own: left to the compiler, the accumulators'
+// shift (below) becomes an in-place multiply-add and a move per value
+__device__ __forceinline__ float fma_to(float w, float x, float a)
+{
+    float d;
+    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(d) : "v"(w), "v"(x), "v"(a));
+    return d;
+}
+__device__ __forceinline__ double fma_to(double w, double x, double a)
+{
+    double d;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(w), "v"(x), "v"(a));
+    return d;
+}
+
+// 16-byte groups covering the x halo, and LDS groups left / right of a row
+template <typename T>
+struct March {
+    static constexpr int V = 16 / sizeof(T);
+    static constexpr int HG = (kR + V - 1) / V;
+    static constexpr int LP = HG + 1, RP = HG;
+    static int row_groups(int gx) { return gx + LP + RP; }
+};
+
+// PART: nx is no multiple of V (a row's last group is partly filled)
+template <typename T, bool HV, bool HZ, bool PART>
+__global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx, int ty, int zchunk)
+{
+    using C = Column<T>;
+    using F = typename C::vec;
+    constexpr int V = C::V, HG = March<T>::HG, LP = March<T>::LP, RP = March<T>::RP;
+    extern __shared__ __align__(16) unsigned char march_smem[];
+    T *lds = reinterpret_cast<T *>(march_smem);
+    const int rs = (gx + LP + RP) * V;         // LDS row stride
+    const int psz = (ty + 2 * kR) * rs;        // one plane
+    // the row tiles of one column are consecutive logical ids -> one XCD
+    const int lid = xcd_remap(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
+                              gridDim.x * gridDim.y * gridDim.z);
+    const int rest = lid / gridDim.x;
+    const int j0 = (lid - rest * gridDim.x) * ty;
+    const int chunk = rest / gridDim.y;
+    const int col = rest - chunk * gridDim.y;
+    const int zs = chunk * zchunk;
+    const int ze = min(p.nz, zs + zchunk);
+    const int nr = min(ty, p.ny - j0);         // rows of this block
+    const int tid = threadIdx.x;
+    const int row = tid / gx, g = tid - row * gx;
+    const int x0 = g * V;
+    const int rem = p.nx - (gx - 1) * V;       // points of a row's last group
+    const bool act = row < nr, last = PART && g == gx - 1;
+    // in-plane byte offsets: my group (loads; whole and partial stores), and
+    // my halo group (rows 0..5 above, 6..11 below the block's rows)
+    const int off = act ? ((j0 + row) * p.nx + x0) * (int)sizeof(T) : kNoRow;
+    const int off_w = last ? kNoRow : off;
+    const int off_2 = last && (V == 2 || (rem & 2)) ? off : kNoRow;
+    const int off_1 = last && V == 4 && (rem & 1) && act ? off + (rem & 2) * (int)sizeof(T) : kNoRow;
+    const int hrow = row < kR ? row : nr + row;
+    const bool hslot = row < 2 * kR;
+    const int hj = hslot ? axis_index(j0 - kR + hrow, p.ny, p.bcy) : -1;
+    const int hoff = hj >= 0 ? (hj * p.nx + x0) * (int)sizeof(T) : kNoRow;
+    const int pbytes = p.nx * p.ny * (int)sizeof(T);
+    const C x(p.x + col * p.ldx, pbytes, p.nz), vc(HV ? p.v : p.x, pbytes, p.nz);
+    const C zc(HZ ? p.z + col * p.ldz : p.x, pbytes, p.nz), oc(p.out + col * p.ldo, pbytes, p.nz);
+    // LDS cells (elements, buffer 0), all 16-byte aligned: my group (threads
+    // past the block's rows read row 0's and write nothing), my halo group.
+    // Cells left of a row and from nx on hold the points at its other end
+    // (periodic x: written by the threads of the first HG and the last LP
+    // groups at wcell) or zeros (Dirichlet).
+    const int own = (kR + (act ? row : 0)) * rs + LP * V + x0;
+    const int hal = hrow * rs + LP * V + x0;
+    const bool lw = g >= gx - (PART ? LP : HG);
+    const bool wrap = act && !p.bcx && (g < HG || lw);
+    const int wcell = lw ? own - p.nx : own + p.nx;
+    auto xplane = [&](int z, int o) {
+        const int za = axis_index(z, p.nz, p.bcz);
+        return x.load(za < 0 ? 0 : za, za < 0 ? kNoRow : o);
+    };
+
+    if (p.bcx) {
+        for (int i = tid; i < 2 * psz; i += blockDim.x) lds[i] = T(0);
+        __syncthreads();
+    }
+
+    F acc[2 * kR];
+#pragma unroll
+    for (int k = 0; k < 2 * kR; k++) acc[k] = F(T(0));
+    // planes zs - 6 .. zs - 1: z contributions to outputs zs .. zs + 5 (acc[6..11])
+    {
+        F pre[kR];
+#pragma unroll
+        for (int j = 0; j < kR; j++) pre[j] = xplane(zs - kR + j, off);
+#pragma unroll
+        for (int k = 0; k < kR; k++)
+#pragma unroll
+            for (int j = k; j < kR; j++) acc[kR + k] += p.wz[k + kR - j] * pre[j];
+    }
+    F xn = x.load(zs, off), hn = x.load(zs, hoff);
+    for (int z = zs; z < ze; z++) {
+        T *pl = lds + ((z - zs) & 1) * psz;
+        const F xv = xn;
+        // consumed after the x / y sums of this plane (z: of output plane z - 6)
+        F vv, zz;
+        if (HV) vv = vc.load(z, off);
+        if (HZ) zz = zc.load(max(z - kR, zs), off);
+        if constexpr (PART) {
+            if (act && !last) *reinterpret_cast<F *>(pl + own) = xv;
+            // element by element: cells of any alignment, the last group's
+            // first rem points only
+#pragma unroll
+            for (int e = 0; e < V - 1; e++)
+                if (act && last && e < rem) pl[own + e] = xv[e];
+#pragma unroll
+            for (int e = 0; e < V; e++)
+                if (wrap && (!last || e < rem)) pl[wcell + e] = xv[e];
+        } else {
+            if (act) *reinterpret_cast<F *>(pl + own) = xv;
+            if (wrap) *reinterpret_cast<F *>(pl + wcell) = xv;
+        }
+        if (hslot) *reinterpret_cast<F *>(pl + hal) = hn;
+        // the next plane's loads, in flight during this plane's sums
+        {
+            const int zn = min(z + 1, ze - 1);
+            xn = x.load(zn, off);
+            hn = x.load(zn, hoff);
+        }
+        __syncthreads();
+        F xy = p.w0 * xv;
+        {
+            T line[(2 * HG + 1) * V];
+#pragma unroll
+            for (int q = 0; q < 2 * HG + 1; q++) {
+                // (a partly filled group takes its own cells back too: past
+                // its points they hold the ones after them)
+                const F w = q == HG && !PART ? xv : *reinterpret_cast<const F *>(pl + own + (q - HG) * V);
+#pragma unroll
+                for (int e = 0; e < V; e++) line[q * V + e] = w[e];
+            }
+#pragma unroll
+            for (int s = 1; s <= kR; s++)
+#pragma unroll
+                for (int e = 0; e < V; e++)
+                    xy[e] += p.wx[s] * (line[HG * V + e - s] + line[HG * V + e + s]);
+        }
+        // the y rows in two halves (all at once would hold 24 registers more)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 1; s <= kR; s++) {
+            const F a = *reinterpret_cast<const F *>(pl + own - s * rs);
+            const F b = *reinterpret_cast<const F *>(pl + own + s * rs);
+            xy += p.wy[s] * (a + b);
+            if (s == kR / 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (HV) xy += p.bdiag * (vv * xv);
+        F done;
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+            done[e] = acc[0][e] + p.wz[kR] * xv[e];
+#pragma unroll
+            for (int k = 0; k < 2 * kR - 1; k++)
+                acc[k][e] = k == kR - 1
+                                ? acc[k + 1][e] + xy[e]
+                                : fma_to(p.wz[k < kR ? kR - 1 - k : k - kR + 1], xv[e], acc[k + 1][e]);
+            acc[2 * kR - 1][e] = p.wz[kR] * xv[e];
+            done[e] *= p.s1;
+            if (HZ) done[e] += p.s2 * zz[e];
+        }
+        const bool out = z - kR >= zs;
+        oc.store(max(z - kR, zs), out ? off_w : kNoRow, done);
+        if (PART) oc.store_part(max(z - kR, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, done, rem);
+    }
+    // planes ze .. ze + 5 finish outputs ze - 6 .. ze - 1 (those from zs on),
+    // three at a time
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        constexpr int H = kR / 2;
+        F pos[H], zt[H];
+#pragma unroll
+        for (int j = 0; j < H; j++) {
+            pos[j] = xplane(ze + h * H + j, off);
+            const int zo = ze - kR + h * H + j;
+            if (HZ) zt[j] = zc.load(max(zo, zs), off);
+        }
+#pragma unroll
+        for (int j = 0; j < H; j++) {
+            // plane ze + h H + j: acc[i] is output ze - 6 + i
+#pragma unroll
+            for (int i = h * H + j; i < kR; i++) acc[i] += p.wz[kR - i + h * H + j] * pos[j];
+            const int zo = ze - kR + h * H + j;
+            F o = p.s1 * acc[h * H + j];
+            if (HZ) o += p.s2 * zt[j];
+            const bool out = zo >= zs;
+            oc.store(max(zo, zs), out ? off_w : kNoRow, o);
+            if (PART) oc.store_part(max(zo, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, o, rem);
+        }
+    }
+}
+
+// Form for small blocks (a 26^3 x 24 block, a single vector): radius 6, V
+// points of one row and one plane per thread, every neighbour loaded straight
+// from L2 with all loads of a thread in flight at once.  What bounds it is one
+// memory latency plus the launch, where the marching forms pay a latency per
+// plane; the 13-fold reads stay in L2 / L1 as long as the block does.
+template <typename T, bool HV, bool HZ>
+__global__ __launch_bounds__(256) void stencil_near(StencilParams<T> p, int gx)
+{
+    using C = Column<T>;
+    using F = typename C::vec;
+    constexpr int V = C::V;
+    // a column's planes are consecutive logical ids -> one XCD
+    const int lid = xcd_remap(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
+                              gridDim.x * gridDim.y * gridDim.z);
+    const int rest = lid / gridDim.x;
+    const int t = (lid - rest * gridDim.x) * 256 + threadIdx.x;
+    const int col = rest / p.nz, z = rest - col * p.nz;
+    const int row = t / gx, g = t - row * gx;
+    const bool act = row < p.ny;
+    // the last group ends at the row's end; of the points it repeats from the
+    // group before it stores none
+    const int x0 = min(g * V, p.nx - V), skip = g * V - x0;
+    const int pb = p.nx * p.ny * (int)sizeof(T);
+    const C x(p.x + col * p.ldx, pb, p.nz), oc(p.out + col * p.ldo, pb, p.nz);
+    const int ro = act ? row * p.nx * (int)sizeof(T) : kNoRow;
+    const int off = act ? ro + x0 * (int)sizeof(T) : kNoRow;
+    const F c = x.load(z, off);
+    F vv, zz;
+    if (HV) vv = C(p.v, pb, p.nz).load(z, off);
+    if (HZ) zz = C(p.z + col * p.ldz, pb, p.nz).load(z, off);
+    T line[V + 2 * kR];
+#pragma unroll
+    for (int e = 0; e < V; e++) line[kR + e] = c[e];
+#pragma unroll
+    for (int s = 1; s <= kR; s++) {
+        int l = x0 - s, r = x0 + V - 1 + s;
+        if (!p.bcx) {
+            l += l < 0 ? p.nx : 0;
+            r -= r >= p.nx ? p.nx : 0;
+        }
+        line[kR - s] = x.load1(z, act && l >= 0 ? ro + l * (int)sizeof(T) : kNoRow);
+        line[kR + V - 1 + s] = x.load1(z, act && r < p.nx ? ro + r * (int)sizeof(T) : kNoRow);
+    }
+    F ya[kR], yb[kR], za[kR], zb[kR];
+#pragma unroll
+    for (int s = 1; s <= kR; s++) {
+        int a = row - s, b = row + s;
+        if (!p.bcy) {
+            a += a < 0 ? p.ny : 0;
+            b -= b >= p.ny ? p.ny : 0;
+        }
+        ya[s - 1] = x.load(z, act && a >= 0 ? off + (a - row) * p.nx * (int)sizeof(T) : kNoRow);
+        yb[s - 1] = x.load(z, act && b < p.ny ? off + (b - row) * p.nx * (int)sizeof(T) : kNoRow);
+    }
+#pragma unroll
+    for (int s = 1; s <= kR; s++) {
+        const int a = axis_index(z - s, p.nz, p.bcz), b = axis_index(z + s, p.nz, p.bcz);
+        za[s - 1] = x.load(max(a, 0), a >= 0 ? off : kNoRow);
+        zb[s - 1] = x.load(max(b, 0), b >= 0 ? off : kNoRow);
+    }
+    F o;
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+        T res = p.w0 * c[e];
+#pragma unroll
+        for (int s = 1; s <= kR; s++) {
+            const T rx = (line[kR + e - s] + line[kR + e + s]) * p.wx[s];
+            const T ry = (ya[s - 1][e] + yb[s - 1][e]) * p.wy[s];
+            const T rz = (za[s - 1][e] + zb[s - 1][e]) * p.wz[s];
+            res += rx + ry + rz;
+        }
+        if (HV) res += p.bdiag * (vv[e] * c[e]);
+        o[e] = p.s1 * res;
+        if (HZ) o[e] += p.s2 * zz[e];
+    }
+    if (skip == 0) {
+        oc.store(z, off, o);
+    } else {
+#pragma unroll
+        for (int e = 1; e < V; e++)
+            if (e >= skip) oc.store1(z, act ? off + e * (int)sizeof(T) : kNoRow, o[e]);
+    }
+}
+
 template <typename T, int TX, int TY, int RY, int NS>
 void launch_ring(sgpu_context *ctx, const StencilParams<T> &p, int ncol)
 {
@@ -574,6 +935,120 @@ void launch_ring(sgpu_context *ctx, const StencilParams<T> &p, int ncol)
     nzc = (ctx->nz + zchunk - 1) / zchunk;
     dim3 grid(tiles, ncol, nzc);
     stencil_ring<T, TX, TY, RY, NS><<<grid, TX * (TY / RY), 0, ctx->stream>>>(p, zchunk);
+}
+
+// The cover of a block by stencil_march.  A CU holds 16 of its waves (128
+// VGPRs), and workgroups land on the four SIMDs evenly only if their waves are
+// a multiple of four (5-wave workgroups: two per CU, 78^3 x 480 FP32 800
+// against 665 us for 4-wave ones), so the rows per workgroup are the most that
+// 256, 512 or 1,024 threads hold, evened out over the tiles; the z-chunks are
+// those with the least rounds x (planes + 8), the 12 planes that every chunk
+// re-reads costing about 8 (measured: 52^3 x 160 FP32 71 us with one chunk, 61
+// with two, 70 with three; 78^3 x 480 FP32 677 / 652 / 748).
+template <typename T>
+sgpu_march_plan plan_march(const sgpu_context *ctx, int ncol)
+{
+    constexpr int V = March<T>::V;
+    const int gx = (ctx->nx + V - 1) / V;
+    sgpu_march_plan plan;
+    if (ctx->nx < 20 || gx > 64 || ctx->nd * (long)sizeof(T) > kNoRow) return plan;
+    double best = 0.0;
+    for (int nt = 256; nt <= 1024; nt *= 2) {
+        const int fit = nt / gx;
+        if (fit < 2 * kR) continue;
+        const int tiles = (ctx->ny + fit - 1) / fit;
+        const int ty = std::max(2 * kR, (ctx->ny + tiles - 1) / tiles);
+        if ((size_t)(ty + 2 * kR) * March<T>::row_groups(gx) * 32 > 64 * 1024) continue;
+        const double slots = (double)ctx->n_cu * (1024 / nt);
+        for (int nzc = 1; nzc <= ctx->nz; nzc++) {
+            const int zc = (ctx->nz + nzc - 1) / nzc;
+            const double blocks = (double)tiles * ncol * ((ctx->nz + zc - 1) / zc);
+            const double cost = std::ceil(blocks / slots) * (zc + 8);
+            if (plan.gx == 0 || cost < 0.98 * best) {
+                best = cost;
+                plan.gx = gx;
+                plan.ty = ty;
+                plan.zchunk = zc;
+            }
+            if (zc <= 2) break;
+        }
+    }
+    return plan;
+}
+
+template <typename T>
+const sgpu_march_plan &march_plan(sgpu_context *ctx, int ncol)
+{
+    const auto key = std::make_pair((int)sizeof(T), ncol);
+    auto it = ctx->march_plans.find(key);
+    if (it == ctx->march_plans.end()) it = ctx->march_plans.emplace(key, plan_march<T>(ctx, ncol)).first;
+    return it->second;
+}
+
+template <typename T>
+void launch_near(sgpu_context *ctx, const StencilParams<T> &p, int ncol)
+{
+    const int gx = (ctx->nx + March<T>::V - 1) / March<T>::V;
+    const dim3 grid((ctx->ny * gx + 255) / 256, ctx->nz, ncol);
+    const bool hv = p.bdiag != T(0), hz = p.z != nullptr;
+    auto go = [&](auto kern) { kern<<<grid, 256, 0, ctx->stream>>>(p, gx); };
+    if (hv && hz) go(stencil_near<T, true, true>);
+    else if (hv) go(stencil_near<T, true, false>);
+    else if (hz) go(stencil_near<T, false, true>);
+    else go(stencil_near<T, false, false>);
+}
+
+template <typename T>
+void launch_march(sgpu_context *ctx, const StencilParams<T> &p, int ncol, const sgpu_march_plan &plan)
+{
+    const int gx = plan.gx, ty = plan.ty, zchunk = plan.zchunk;
+    const int nt = (gx * ty + 63) / 64 * 64;
+    const size_t shm = (size_t)(ty + 2 * kR) * March<T>::row_groups(gx) * 32;
+    const dim3 grid((ctx->ny + ty - 1) / ty, ncol, (ctx->nz + zchunk - 1) / zchunk);
+    const bool hv = p.bdiag != T(0), hz = p.z != nullptr;
+    auto go = [&](auto kern) { kern<<<grid, nt, shm, ctx->stream>>>(p, gx, ty, zchunk); };
+    if (ctx->nx % March<T>::V) {
+        if (hv && hz) go(stencil_march<T, true, true, true>);
+        else if (hv) go(stencil_march<T, true, false, true>);
+        else if (hz) go(stencil_march<T, false, true, true>);
+        else go(stencil_march<T, false, false, true>);
+    } else {
+        if (hv && hz) go(stencil_march<T, true, true, false>);
+        else if (hv) go(stencil_march<T, true, false, false>);
+        else if (hz) go(stencil_march<T, false, true, false>);
+        else go(stencil_march<T, false, false, false>);
+    }
+}
+
+// Largest block stencil_near takes: below it one latency beats the marching
+// form's one per plane (FP64 52^3 x 1, 1.1 MB: 6.1 against 7.4 us; FP32
+// 26^3 x 24, 1.7 MB: 7.1 / 8.7; FP64 26^3 x 24, 3.4 MB: 9.9 / 10.6), above it
+// the repeated reads cost more (FP64 80^3 x 1, 4.1 MB: 11.4 / 10.9; FP32
+// 36^3 x 24, 4.5 MB: 14.1 / 11.4; FP64 128^3 x 1: 26.0 / 16.7).
+constexpr long kNearBytes = 3600000;
+
+// Launches stencil_near or stencil_march where they apply (false: the tiles
+// below).  Grids of fewer than 16 planes, which no SCF or Poisson grid has,
+// keep the tuned tiles, whose bits do not depend on the tile.
+template <typename T>
+bool launch_vec(sgpu_context *ctx, const StencilParams<T> &p, int ncol, int cfg)
+{
+    if (cfg >= 0 && cfg < 20) return false;
+    const bool near_fits = ctx->nx >= 20 && ctx->nd * (long)sizeof(T) <= kNoRow;
+    if (cfg < 0) {
+        if (ctx->nz < 16) return false;
+        cfg = near_fits && ctx->nd * (long)ncol * (long)sizeof(T) <= kNearBytes ? 21 : 20;
+    }
+    if (cfg == 21 && near_fits) {
+        launch_near<T>(ctx, p, ncol);
+    } else {
+        const sgpu_march_plan &plan = march_plan<T>(ctx, ncol);
+        if (plan.gx == 0) return false;
+        launch_march<T>(ctx, p, ncol, plan);
+        cfg = 20;
+    }
+    ctx->tile_choice[std::make_pair((int)sizeof(T), ncol)] = cfg;
+    return true;
 }
 
 // min_chunk: fewest z-planes per block (each chunk re-reads 2 x 6 planes)
@@ -724,6 +1199,11 @@ int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, 
     }
     if (allow_tiled && ctx->fdn == kR) {
         int cfg = ctx->stencil_cfg;
+        if (launch_vec<T>(ctx, p, ncol, cfg)) {
+            SGPU_HIP(hipGetLastError());
+            return SGPU_OK;
+        }
+        if (cfg >= 20) cfg = -1;  // forced where it does not apply
         if (cfg < 0) {
             const auto key = std::make_pair((int)sizeof(T), ncol);
             auto it = ctx->tile_choice.find(key);
@@ -777,13 +1257,22 @@ extern "C" int sgpu_stencil_tile(const sgpu_context *ctx, int dtype, int ncol, i
         return SGPU_ERR_ARG;
     }
     int cfg = ctx->stencil_cfg;
-    if (cfg < 0) {
-        auto it = ctx->tile_choice.find(std::make_pair(dtype == SGPU_F64 ? 8 : 4, ncol));
+    if (cfg < 0 || cfg >= 20) {
+        const auto key = std::make_pair(dtype == SGPU_F64 ? 8 : 4, ncol);
+        auto it = ctx->tile_choice.find(key);
         if (it == ctx->tile_choice.end()) {
             *tx = *ty = *ry = 0;
             return SGPU_OK;
         }
         cfg = it->second;
+        if (cfg >= 20) {  // whole rows, one row per thread
+            const int gx = (ctx->nx + 16 / key.first - 1) / (16 / key.first);
+            auto pl = ctx->march_plans.find(key);
+            *tx = ctx->nx;
+            *ty = cfg == 20 && pl != ctx->march_plans.end() ? pl->second.ty : std::max(1, 256 / gx);
+            *ry = 1;
+            return SGPU_OK;
+        }
     }
     static const int shape[15][3] = {{32, 16, 2}, {32, 32, 4}, {64, 16, 4}, {32, 32, 8},
                                      {64, 32, 8}, {32, 16, 2}, {32, 8, 2},  {32, 32, 2},
@@ -806,13 +1295,19 @@ extern "C" int sgpu_stencil_kernel(const sgpu_context *ctx, int dtype, int ncol,
     }
     SGPU_CHECK(sgpu_stencil_tile(ctx, dtype, ncol, &tx, &ty, &ry));
     int cfg = ctx->stencil_cfg;
-    if (cfg < 0) {
+    if (cfg < 0 || cfg >= 20) {
         auto it = ctx->tile_choice.find(std::make_pair(dtype == SGPU_F64 ? 8 : 4, ncol));
         cfg = it == ctx->tile_choice.end() ? 0 : it->second;
     }
     const char *t = dtype == SGPU_F64 ? "double" : "float";
+    // (of the vector forms the recurrence's instance: Veff and z terms)
     if (tx == 0)
         name[0] = 0;
+    else if (cfg == 20)
+        snprintf(name, len, "stencil_march<%s,true,true,%s>", t,
+                 ctx->nx % (dtype == SGPU_F64 ? 2 : 4) ? "true" : "false");
+    else if (cfg == 21)
+        snprintf(name, len, "stencil_near<%s,true,true>", t);
     else if ((cfg == 13 || cfg == 14) && dtype != SGPU_F64 && ctx->nx == tx)
         snprintf(name, len, "stencil_rows<%d,%d,%d>", tx, ty, ry);
     else if ((cfg == 5 || cfg == 6) && dtype != SGPU_F64)

@@ -129,6 +129,43 @@ def test_stencil_ring_fp32(gpu, oracle_mod, monkeypatch, cfg, n, bc, ncol):
     assert rel_err(y64, o.lap_plus_diag(x, -0.5, 1.0, 0.4, veff)) < 1e-13
 
 
+@pytest.mark.parametrize("form", [20, 21, None])
+@pytest.mark.parametrize("n,bc,ncol", [
+    ((20, 16, 16), (0, 0, 0), 3),    # smallest row, one tile
+    ((21, 17, 16), (0, 1, 0), 2),    # one point in a row's last group (FP32 and FP64)
+    ((23, 30, 19), (1, 0, 1), 5),    # three points, Dirichlet x
+    ((78, 27, 18), (0, 0, 1), 3),    # two points, several row tiles, the last one partial
+    ((33, 6, 40), (0, 0, 0), 1),     # fewer rows than a tile's halo, z-chunks
+    ((128, 13, 16), (1, 1, 1), 2),   # longest FP64 row
+    ((256, 14, 16), (0, 0, 0), 1),   # longest FP32 row (FP64 takes the tiles)
+])
+def test_stencil_vector_forms(gpu, oracle_mod, monkeypatch, form, n, bc, ncol):
+    """The 16-bytes-per-thread stencils (20: marching, 21: for small blocks)
+    and the default choice between them: the first application (no z term) and
+    the in-place recurrence (out aliasing z), against the oracle's filter.
+    FP64: sums of 37 products, 1e-13 as for the tiles; FP32: two chained
+    applications of rounding 2^-24 per product, 3e-6 as for the tiles."""
+    if form is None:
+        monkeypatch.delenv("SPARC_AMD_STENCIL_TILE", raising=False)
+    else:
+        monkeypatch.setenv("SPARC_AMD_STENCIL_TILE", str(form))
+    g, veff, nl, rng = small_case(n=n, bc=bc, seed=90 + n[0])
+    o = oracle_mod.Oracle(g, veff)
+    x = rng.uniform(-0.5, 0.5, (g.nd, ncol)).astype(np.float32).astype(np.float64)
+    yo, po = o.chebyshev_filter(x, 3, 2.0, 90.0, -3.0)
+    for dt, tol in ((gpu.F64, 1e-13), (gpu.F32, 3e-6)):
+        with gpu.Context(g) as ctx:
+            ctx.set_veff(veff)
+            bx = ctx.block(ncol, dt).upload(x)
+            by = ctx.block(ncol, dt).fill_uniform(7, -1.0, 1.0)  # stale output
+            ctx.chebyshev_filter_dev(bx, by, 3, 2.0, 90.0, -3.0)
+            y, prev = by.download(), bx.download()
+            name = ctx.stencil_kernel(dt, ncol)
+        if n[0] <= (128 if dt == gpu.F64 else 256):
+            assert name.startswith({20: "stencil_march<", 21: "stencil_near<", None: "stencil_"}[form]), name
+        assert rel_err(y, yo) < tol and rel_err(prev, po) < tol
+
+
 @pytest.mark.parametrize("order", [2, 4, 8, 16])
 def test_lap_other_orders(gpu, oracle_mod, order):
     g, veff, nl, rng = small_case(n=(12, 11, 10), order=order, seed=2)
