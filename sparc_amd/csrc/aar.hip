@@ -4,12 +4,16 @@
 // src/mixing.c:48-139, poisson_residual src/lapVecRoutines.c:69-79,
 // Jacobi_preconditioner src/electrostatics.c:1682-1699).
 //
-// Per Richardson iteration the built-in path runs two kernels: one fused
-// pass (Jacobi f = -r/d, history columns X/F, x_old/f_old, x += omega f)
-// and the residual stencil r = b + (Lap + c) x (the b add is fused into the
-// stencil epilogue).  Anderson steps add one pass computing F'F and F'f
-// together and one update pass; the m x m minimum-norm solve is done on the
-// host in FP64.
+// The last m + 1 iterates x_k and preconditioned residuals f_k are kept as they
+// are, in two rings; the history differences that Anderson mixing takes are
+// formed where they are used.  With the built-in residual and preconditioner a
+// Richardson iteration is then one launch (sgpu_launch_aar_step: the stencil
+// with f = jac r and x + omega f in its epilogue; x twice, b, f and the new x
+// are 5 vectors moved, against 15 for a residual stencil followed by a pass
+// that kept r, x_old, f_old and two difference columns).  Anderson steps add
+// one pass for F'F and F'f together and one update pass; the m x m
+// minimum-norm solve is done on the host in FP64.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -19,24 +23,106 @@ namespace {
 
 constexpr int kAarMaxM = 8;
 
-// f = jac * r (when jac != 0; otherwise f is given); history and Richardson.
-__global__ void aar_fused(const double *__restrict__ r, double *__restrict__ f, double jac,
-                          double *__restrict__ x, double *__restrict__ x_old,
-                          double *__restrict__ f_old, double *__restrict__ Xh,
-                          double *__restrict__ Fh, int store_hist, double omega, long n)
+// f = jac r (when jac != 0; otherwise f is given) and, when xn is given,
+// xn = x + omega f.
+__global__ void aar_step(const double *__restrict__ r, double *__restrict__ f, double jac,
+                         const double *__restrict__ x, double *__restrict__ xn, double omega, long n)
 {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const double fi = jac != 0.0 ? jac * r[i] : f[i];
     if (jac != 0.0) f[i] = fi;
-    const double xi = x[i];
-    if (store_hist) {
-        Xh[i] = xi - x_old[i];
-        Fh[i] = fi - f_old[i];
+    if (xn) xn[i] = x[i] + omega * fi;
+}
+
+struct AarCoeff {
+    double g[kAarMaxM];
+};
+
+// The ring vectors v_k, v_(k-1), ... by age.
+struct AarRing {
+    const double *v[kAarMaxM + 1];
+};
+
+// Sums over the block's share of F'F (upper triangle) and F'f into partial,
+// from the NV accumulators of every thread.
+template <int NV>
+__device__ __forceinline__ void gram_partial(const double (&acc)[NV], double *__restrict__ partial)
+{
+    __shared__ double sh[4][NV];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        double s = acc[k];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (lane == 0) sh[wave][k] = s;
     }
-    x_old[i] = xi;
-    f_old[i] = fi;
-    if (omega != 0.0) x[i] = xi + omega * fi;
+    __syncthreads();
+    for (int k = threadIdx.x; k < NV; k += 256)
+        partial[(long)blockIdx.x * NV + k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+}
+
+// Recorded solves (training pairs) keep one fixed order of operations, so that
+// a network trained on them does not depend on the forms chosen for speed: the
+// columns of aar_gram / aar_update_cols are the history differences formed by
+// aar_columns, in the order d % m of the steps d they come from.
+__global__ void aar_columns(AarRing x, AarRing f, int m, int rot, long ld, double *__restrict__ Xh,
+                            double *__restrict__ Fh, long n)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    for (int j = 0; j < m; j++) {
+        const long at = (long)((rot + m - j) % m) * ld + i;  // age j
+        Xh[at] = x.v[j][i] - x.v[j + 1][i];
+        Fh[at] = f.v[j][i] - f.v[j + 1][i];
+    }
+}
+
+// xn = x - Xh G + beta (f - Fh G)
+__global__ void aar_update_cols(double *xn, const double *x, const double *__restrict__ f,
+                                const double *__restrict__ Xh, const double *__restrict__ Fh, long ldh,
+                                int m, AarCoeff G, double beta, long n)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double xw = x[i], fw = f[i];
+#pragma unroll
+    for (int a = 0; a < kAarMaxM; a++) {
+        if (a < m) {
+            xw -= Xh[a * ldh + i] * G.g[a];
+            fw -= Fh[a * ldh + i] * G.g[a];
+        }
+    }
+    xn[i] = xw + beta * fw;
+}
+
+// The same sums as aar_gram for the columns F_j = f_(k-j) - f_(k-j-1), j < m.
+// Bound by reading m + 1 vectors; four workgroups per CU (with one, as
+// aar_gram has, too few bytes were in flight: 128^3, m = 7, 44 -> 33 us).
+template <int M>
+__global__ __launch_bounds__(256) void aar_gram_ring(AarRing f, int m, long n,
+                                                     double *__restrict__ partial)
+{
+    constexpr int NV = M * (M + 1) / 2 + M;
+    double acc[NV];
+#pragma unroll
+    for (int k = 0; k < NV; k++) acc[k] = 0.0;
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+        double v[M + 1];
+#pragma unroll
+        for (int a = 0; a <= M; a++) v[a] = a <= m ? f.v[a][i] : 0.0;
+        const double fi = v[0];
+#pragma unroll
+        for (int a = 0; a < M; a++) v[a] = a < m ? v[a] - v[a + 1] : 0.0;
+        int k = 0;
+#pragma unroll
+        for (int a = 0; a < M; a++)
+#pragma unroll
+            for (int b = a; b < M; b++) acc[k++] += v[a] * v[b];
+#pragma unroll
+        for (int a = 0; a < M; a++) acc[k++] += v[a] * fi;
+    }
+    gram_partial<NV>(acc, partial);
 }
 
 // Partial sums of F'F (upper triangle, m(m+1)/2 values) and F'f (m values).
@@ -62,17 +148,7 @@ __global__ __launch_bounds__(256) void aar_gram(const double *__restrict__ F, lo
 #pragma unroll
         for (int a = 0; a < M; a++) acc[k++] += v[a] * fi;
     }
-    __shared__ double sh[4][NV];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < NV; k++) {
-        double s = acc[k];
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-        if (lane == 0) sh[wave][k] = s;
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < NV; k += 256)
-        partial[(long)blockIdx.x * NV + k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+    gram_partial<NV>(acc, partial);
 }
 
 // One wave per Gram value: lane l sums the partials l, l + 64, ... in order,
@@ -87,25 +163,30 @@ __global__ __launch_bounds__(64) void aar_gram_final(const double *__restrict__ 
     if (lane == 0) out[k] = s;
 }
 
-// x = x_old - X G + beta (f - F G)
-__global__ void aar_anderson_update(double *__restrict__ x, const double *__restrict__ x_old,
-                                    const double *__restrict__ f, const double *__restrict__ Xh,
-                                    const double *__restrict__ Fh, long ldh, int m, double g0,
-                                    double g1, double g2, double g3, double g4, double g5,
-                                    double g6, double g7, double beta, long n)
+// xn = x_k - X G + beta (f_k - F G) with F_j = f_(k-j) - f_(k-j-1) and
+// X_j = x_(k-j) - x_(k-j-1) where bit j of xdiff is set (step k - j - 1 was an
+// Anderson one), omega f_(k-j-1) otherwise (a Richardson step moved x by just
+// that), which needs no x vectors.  xn may be the oldest x.
+template <int M>
+__global__ __launch_bounds__(256) void aar_update(double *xn, AarRing x, AarRing f, int m,
+                                                  unsigned xdiff, AarCoeff G, double omega, double beta,
+                                                  long n)
 {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double g[kAarMaxM] = {g0, g1, g2, g3, g4, g5, g6, g7};
-    double xw = x_old[i], fw = f[i];
+    double v[M + 1];
 #pragma unroll
-    for (int a = 0; a < kAarMaxM; a++) {
+    for (int a = 0; a <= M; a++) v[a] = a <= m ? f.v[a][i] : 0.0;
+    double xw = x.v[0][i], fw = v[0];
+#pragma unroll
+    for (int a = 0; a < M; a++) {
         if (a < m) {
-            xw -= Xh[a * ldh + i] * g[a];
-            fw -= Fh[a * ldh + i] * g[a];
+            const double d = (xdiff >> a & 1) ? x.v[a][i] - x.v[a + 1][i] : omega * v[a + 1];
+            xw -= d * G.g[a];
+            fw -= (v[a] - v[a + 1]) * G.g[a];
         }
     }
-    x[i] = xw + beta * fw;
+    xn[i] = xw + beta * fw;
 }
 
 // Symmetric eigendecomposition by cyclic Jacobi rotations (m <= 8).
@@ -171,6 +252,21 @@ void anderson_coeff(int m, const double *FtF, const double *Ftf, double *G)
     }
 }
 
+// The unpacked sums of a Gram pass (upper triangle of M x M, then F'f) on the
+// host: G = pinv(F'F) F'f for the first m columns.
+template <int M>
+static void gram_solve(const double *sums, int m, double *G)
+{
+    double FtF[kAarMaxM * kAarMaxM], Ftf[kAarMaxM];
+    int k = 0;
+    for (int a = 0; a < M; a++)
+        for (int bb = a; bb < M; bb++, k++)
+            if (a < m && bb < m) FtF[a + bb * m] = FtF[bb + a * m] = sums[k];
+    for (int a = 0; a < M; a++, k++)
+        if (a < m) Ftf[a] = sums[k];
+    anderson_coeff(m, FtF, Ftf, G);
+}
+
 // G = pinv(F'F) F'f for device F (n x m, column stride ldf) and f: one pass
 // computes F'F and F'f together, the m x m solve runs on the host in FP64.
 int sgpu_anderson_coeff_dev(sgpu_context *ctx, const double *F, long ldf, int m, const double *f,
@@ -191,27 +287,26 @@ int sgpu_anderson_coeff_dev(sgpu_context *ctx, const double *F, long ldf, int m,
     SGPU_HIP(hipMemcpyAsync(ctx->host_red, out, nv * sizeof(double), hipMemcpyDeviceToHost,
                             ctx->stream));
     SGPU_HIP(hipStreamSynchronize(ctx->stream));
-    double FtF[kAarMaxM * kAarMaxM], Ftf[kAarMaxM];
-    int k = 0;
-    for (int a = 0; a < kAarMaxM; a++)
-        for (int bb = a; bb < kAarMaxM; bb++, k++)
-            if (a < m && bb < m) FtF[a + bb * m] = FtF[bb + a * m] = ctx->host_red[k];
-    for (int a = 0; a < kAarMaxM; a++, k++)
-        if (a < m) Ftf[a] = ctx->host_red[k];
-    anderson_coeff(m, FtF, Ftf, G);
+    gram_solve<kAarMaxM>(ctx->host_red, m, G);
     return SGPU_OK;
 }
 
-// x = xk - X G + beta (f - F G) on device vectors (history stride ldh).
-int sgpu_anderson_update_dev(sgpu_context *ctx, double *x, const double *xk, const double *f,
-                             const double *Xh, const double *Fh, long ldh, int m, const double *G,
-                             double beta, long n)
+// G for the ring's differences (aar_gram_ring).
+template <int M>
+static int ring_coeff(sgpu_context *ctx, const AarRing &f, int m, long n, double *G)
 {
-    double g[kAarMaxM] = {0};
-    for (int a = 0; a < m && a < kAarMaxM; a++) g[a] = G[a];
-    aar_anderson_update<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(
-        x, xk, f, Xh, Fh, ldh, m, g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7], beta, n);
+    constexpr int nv = M * (M + 1) / 2 + M;
+    const int blocks = (int)std::min<long>((n + 255) / 256, 4L * ctx->n_cu);
+    double *partial = nullptr;
+    SGPU_CHECK(sgpu_reduce_buf(ctx, (size_t)blocks * nv + nv, &partial));
+    double *out = partial + (size_t)blocks * nv;
+    aar_gram_ring<M><<<blocks, 256, 0, ctx->stream>>>(f, m, n, partial);
+    aar_gram_final<<<nv, 64, 0, ctx->stream>>>(partial, blocks, nv, out);
     SGPU_HIP(hipGetLastError());
+    SGPU_HIP(hipMemcpyAsync(ctx->host_red, out, nv * sizeof(double), hipMemcpyDeviceToHost,
+                            ctx->stream));
+    SGPU_HIP(hipStreamSynchronize(ctx->stream));
+    gram_solve<M>(ctx->host_red, m, G);
     return SGPU_OK;
 }
 
@@ -227,8 +322,11 @@ int sgpu_aar_device(sgpu_context *ctx, sgpu_res_fn res, sgpu_precond_fn precond,
     }
     const long n = N;
     const long ld = ctx->ld;
-    // r, x_old, f, f_old, X (m), F (m): cached on the context
-    const size_t elems = (size_t)(4 + 2 * m) * ld;
+    // r and the rings of x and f (recorded solves: also their differences):
+    // cached on the context
+    const bool recording = rec && rec->fn;
+    const int S = m + 1;
+    const size_t elems = (size_t)(1 + 2 * S + (recording ? 2 * m : 0)) * ld;
     if (elems > ctx->aar_elems) {
         SGPU_HIP(hipStreamSynchronize(ctx->stream));
         if (ctx->aar_mem) SGPU_HIP(hipFree(ctx->aar_mem));
@@ -237,66 +335,108 @@ int sgpu_aar_device(sgpu_context *ctx, sgpu_res_fn res, sgpu_precond_fn precond,
         SGPU_HIP(hipMalloc((void **)&ctx->aar_mem, elems * sizeof(double)));
         ctx->aar_elems = elems;
     }
-    double *mem = ctx->aar_mem;
-    double *r = mem, *x_old = mem + ld, *f = mem + 2 * ld, *f_old = mem + 3 * ld;
-    double *Xh = mem + 4 * ld, *Fh = Xh + (long)m * ld;
+    double *r = ctx->aar_mem;
+    auto X = [&](int k) { return ctx->aar_mem + (long)(1 + k % S) * ld; };
+    auto F = [&](int k) { return ctx->aar_mem + (long)(1 + S + k % S) * ld; };
     const unsigned nb = (unsigned)((n + 255) / 256);
-    int it = 0;
-    double rnorm = 0.0, bnorm = 0.0;
     const double dsum = ctx->d2x[0] + ctx->d2y[0] + ctx->d2z[0] + c;
     const double jac = -1.0 / (std::fabs(dsum) < 1e-14 ? 1.0 : dsum);
+    auto anderson = [&](int k) { return k > 0 && (k + 1) % p == 0; };
+    // the step in one launch needs no r of its own
+    bool fused = !res && !precond && !recording;
 
-    auto residual = [&]() -> int {
+    // r_k, and when fused f_k and (Richardson steps) x_(k+1) with it
+    auto evaluate = [&](int k) -> int {
+        sgpu_tmark t;
+        SGPU_CHECK(sgpu_tbegin(ctx, &t));
+        if (fused) {
+            bool done = false;
+            SGPU_CHECK(sgpu_launch_aar_step(ctx, c, X(k), b, F(k), anderson(k) ? nullptr : X(k + 1),
+                                            jac, omega, &done));
+            if (done) {
+                SGPU_CHECK(sgpu_tend(ctx, &t, "aar_residual"));
+                return SGPU_OK;
+            }
+            fused = false;
+        }
         if (res) {
-            res(user, N, c, x, b, r);
+            res(user, N, c, X(k), b, r);
         } else {
             // r = b + (Lap + c) x
-            sgpu_tmark t;
-            SGPU_CHECK(sgpu_tbegin(ctx, &t));
-            SGPU_CHECK(sgpu_launch_stencil(ctx, SGPU_F64, 1, 1.0, 0.0, c, nullptr, x, ld, r, ld, b,
-                                           ld, 1.0, 1.0, true));
+            SGPU_CHECK(sgpu_launch_stencil(ctx, SGPU_F64, 1, 1.0, 0.0, c, nullptr, X(k), ld, r, ld, b,
+                                           ld, 1.0, 1.0, true, true, recording));
             SGPU_CHECK(sgpu_tend(ctx, &t, "aar_residual"));
         }
-        if (rec && rec->fn) rec->fn(rec->user, x, r);
+        if (recording) rec->fn(rec->user, X(k), r);
         return SGPU_OK;
     };
-    SGPU_HIP(hipMemsetAsync(Xh, 0, 2 * (size_t)m * ld * sizeof(double), ctx->stream));
-    SGPU_HIP(hipMemcpyAsync(x_old, x, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-    const double *pa[1] = {b}, *pb[1] = {b};
-    SGPU_CHECK(sgpu_dot_many(ctx, N, 1, pa, pb, &bnorm));
+    // |r_k| from what evaluate(k) left
+    auto residual_norm = [&](int k, double *norm) -> int {
+        const double *v[1] = {fused ? F(k) : r};
+        SGPU_CHECK(sgpu_dot_many(ctx, N, 1, v, v, norm));
+        *norm = std::sqrt(*norm) / (fused ? std::fabs(jac) : 1.0);
+        return SGPU_OK;
+    };
+    SGPU_HIP(hipMemcpyAsync(X(0), x, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+    int it = 0, cur = 0, normed = -1;  // cur: the newest x; normed: the x of rnorm
+    double rnorm = 0.0, bnorm = 0.0;
+    const double *pb[1] = {b};
+    SGPU_CHECK(sgpu_dot_many(ctx, N, 1, pb, pb, &bnorm));
     bnorm = std::sqrt(bnorm);
-    SGPU_CHECK(residual());
+    SGPU_CHECK(evaluate(0));
     const double atol = tol * bnorm;
     rnorm = atol + 1.0;
     while (rnorm > atol && it < max_iter) {
-        const bool anderson = ((it + 1) % p == 0) && it > 0;
-        const int ih = it > 0 ? (it - 1) % m : 0;
-        if (precond) precond(user, N, c, r, f);
-        aar_fused<<<nb, 256, 0, ctx->stream>>>(r, f, precond ? 0.0 : jac, x, x_old, f_old,
-                                               Xh + (long)ih * ld, Fh + (long)ih * ld,
-                                               it > 0 ? 1 : 0, anderson ? 0.0 : omega, n);
-        SGPU_HIP(hipGetLastError());
-        if (anderson) {
-            double G[kAarMaxM] = {0};
-            SGPU_CHECK(sgpu_anderson_coeff_dev(ctx, Fh, ld, m, f, n, G));
-            SGPU_CHECK(sgpu_anderson_update_dev(ctx, x, x_old, f, Xh, Fh, ld, m, G, beta, n));
-            SGPU_CHECK(residual());
-            pa[0] = r; pb[0] = r;
-            SGPU_CHECK(sgpu_dot_many(ctx, N, 1, pa, pb, &rnorm));
-            rnorm = std::sqrt(rnorm);
+        const bool and_step = anderson(it);
+        if (!fused) {
+            if (precond) precond(user, N, c, r, F(it));
+            if (!precond || !and_step)
+                aar_step<<<nb, 256, 0, ctx->stream>>>(r, F(it), precond ? 0.0 : jac, X(it),
+                                                      and_step ? nullptr : X(it + 1), omega, n);
+            SGPU_HIP(hipGetLastError());
+        }
+        if (and_step) {
+            const int nh = std::min(it, m);
+            AarRing xr, fr;
+            AarCoeff G = {{0}};
+            unsigned xdiff = 0;
+            for (int j = 0; j <= kAarMaxM; j++) {
+                xr.v[j] = X(it - std::min(j, nh));
+                fr.v[j] = F(it - std::min(j, nh));
+                if (j < nh && anderson(it - j - 1)) xdiff |= 1u << j;
+            }
+            if (recording) {
+                double *Xh = ctx->aar_mem + (long)(1 + 2 * S) * ld, *Fh = Xh + (long)m * ld;
+                aar_columns<<<nb, 256, 0, ctx->stream>>>(xr, fr, m, (it - 1) % m, ld, Xh, Fh, n);
+                SGPU_CHECK(sgpu_anderson_coeff_dev(ctx, Fh, ld, m, F(it), n, G.g));
+                aar_update_cols<<<nb, 256, 0, ctx->stream>>>(X(it + 1), X(it), F(it), Xh, Fh, ld, m, G,
+                                                             beta, n);
+            } else if (m <= 7) {
+                SGPU_CHECK(ring_coeff<7>(ctx, fr, nh, n, G.g));
+                aar_update<7><<<nb, 256, 0, ctx->stream>>>(X(it + 1), xr, fr, nh, xdiff, G, omega, beta, n);
+            } else {
+                SGPU_CHECK(ring_coeff<kAarMaxM>(ctx, fr, nh, n, G.g));
+                aar_update<kAarMaxM><<<nb, 256, 0, ctx->stream>>>(X(it + 1), xr, fr, nh, xdiff, G, omega,
+                                                                  beta, n);
+            }
+            SGPU_HIP(hipGetLastError());
+        }
+        cur = it + 1;
+        SGPU_CHECK(evaluate(cur));
+        if (and_step) {
+            SGPU_CHECK(residual_norm(cur, &rnorm));
+            normed = cur;
             // diverged (not finite, or 1e6 x the right-hand side's norm, which
             // no converging solve reaches): reported as not converged at once
             // instead of after max_iter iterations
             if (!std::isfinite(rnorm) || (bnorm > 0 && rnorm > 1e6 * bnorm)) break;
-        } else {
-            SGPU_CHECK(residual());
         }
         it++;
     }
-    double r2 = 0.0;
-    pa[0] = r; pb[0] = r;
-    SGPU_CHECK(sgpu_dot_many(ctx, N, 1, pa, pb, &r2));
-    if (relres) *relres = bnorm > 0 ? std::sqrt(r2) / bnorm : 0.0;
+    double rlast = rnorm;
+    if (normed != cur) SGPU_CHECK(residual_norm(cur, &rlast));
+    SGPU_HIP(hipMemcpyAsync(x, X(cur), n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+    if (relres) *relres = bnorm > 0 ? rlast / bnorm : 0.0;
     if (iters) *iters = it;
     return (!std::isfinite(rnorm) || rnorm > atol) ? SGPU_NOT_CONVERGED : SGPU_OK;
 }

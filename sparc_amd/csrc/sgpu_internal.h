@@ -187,7 +187,7 @@ struct sgpu_context {
     double *red_buf = nullptr;      // reduction partials
     size_t red_elems = 0;
     double *host_red = nullptr;     // pinned host mirror of small results
-    double *aar_mem = nullptr;      // AAR work vectors (r, x_old, f, f_old, X, F)
+    double *aar_mem = nullptr;      // AAR work vectors (r, the last m + 1 x and f)
     size_t aar_elems = 0;
 
     bool timing = false;
@@ -243,10 +243,16 @@ int sgpu_tdc(sgpu_context *ctx, int n, double *dD, const double *dE, double *dZ,
 // out = s1 * ((a Lap + bdiag diag(v) + c) x) + s2 * z, per column (z may be null).
 // may_tune = false never times tile shapes (the timing allocates a temporary
 // output): a shape already chosen for (dtype, ncol) is used, else 32x16x2.
+// tiles_only: the tiled kernels' order of operations whatever the size.
 int sgpu_launch_stencil(sgpu_context *ctx, int dtype, int ncol, double a, double bdiag, double c,
                         const void *v, const void *x, long ldx, void *out, long ldo,
                         const void *z, long ldz, double s1, double s2, bool allow_tiled,
-                        bool may_tune = true);
+                        bool may_tune = true, bool tiles_only = false);
+// One AAR evaluation in one launch: f = jac (b + (Lap + c) x) and, when xn is
+// given, xn = x + omega f (FP64, one vector).  *done is false, and nothing was
+// launched, where the vector stencils do not apply.
+int sgpu_launch_aar_step(sgpu_context *ctx, double c, const double *x, const double *b, double *f,
+                         double *xn, double jac, double omega, bool *done);
 // ---- nonlocal.hip ----
 void sgpu_free_nonlocal(sgpu_nonlocal &nl);
 // Scratch bytes sgpu_launch_vnl takes for ncol columns of dtype.
@@ -277,9 +283,6 @@ void sgpu_unet_orphan(sgpu_unet *u);
 void anderson_coeff(int m, const double *FtF, const double *Ftf, double *G);
 int sgpu_anderson_coeff_dev(sgpu_context *ctx, const double *F, long ldf, int m, const double *f,
                             long n, double *G);
-int sgpu_anderson_update_dev(sgpu_context *ctx, double *x, const double *xk, const double *f,
-                             const double *Xh, const double *Fh, long ldh, int m, const double *G,
-                             double beta, long n);
 // AAR on device vectors (x in/out, b), returns SGPU_OK / SGPU_NOT_CONVERGED / error.
 // Optional observer of the AAR iterates: fn(user, x, r) after every residual
 // evaluation (r = b + (Lap + c) x), on the context's stream.

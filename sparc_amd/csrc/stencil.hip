@@ -11,10 +11,10 @@
 // :536-577); Dirichlet halos read zero.
 //
 // Kernels:
-//  * stencil_march<T, HV, HZ, PART>: radius 6, the default for blocks above
+//  * stencil_march<T, HV, HZ, PART, STEP>: radius 6, the default for blocks above
 //    3.6 MB: whole x-rows, 16 bytes per thread, a block of rows marching along z
 //    with the z sums pending in registers.
-//  * stencil_near<T, HV, HZ>: radius 6, the default for smaller blocks: every
+//  * stencil_near<T, HV, HZ, STEP>: radius 6, the default for smaller blocks: every
 //    neighbour straight from L2.
 //  * stencil_tiled<T, TX, TY, RY>: radius 6.  A TX x TY tile of the x-y plane
 //    (plus a 6-deep halo) is staged in LDS per z-plane while the block marches
@@ -24,6 +24,8 @@
 //    tiled kernel, with no x halo reads and the y halo read kR planes early.
 //  * stencil_direct<T, R>: one thread per point, all 6R+1 loads from global;
 //    used for other FD orders and as the independent cross-check.
+#include <type_traits>
+
 #include "sgpu_internal.h"
 
 namespace {
@@ -41,6 +43,9 @@ struct StencilParams {
     T w0;     // a (D2x0 + D2y0 + D2z0) + c
     T bdiag;  // coefficient of v (0 -> no diagonal term)
     T s1, s2;
+    T *xn;     // stencil_march / stencil_near with STEP: xn = x + omega out
+    long ldn;
+    T omega;
 };
 
 // Index along one axis with the halo convention; returns -1 for a Dirichlet
@@ -668,8 +673,10 @@ struct March {
     static int row_groups(int gx) { return gx + LP + RP; }
 };
 
-// PART: nx is no multiple of V (a row's last group is partly filled)
-template <typename T, bool HV, bool HZ, bool PART>
+// PART: nx is no multiple of V (a row's last group is partly filled); STEP:
+// also xn = x + omega out (the Richardson step of AAR, whose out is the
+// preconditioned residual)
+template <typename T, bool HV, bool HZ, bool PART, bool STEP>
 __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx, int ty, int zchunk)
 {
     using C = Column<T>;
@@ -707,6 +714,7 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
     const int pbytes = p.nx * p.ny * (int)sizeof(T);
     const C x(p.x + col * p.ldx, pbytes, p.nz), vc(HV ? p.v : p.x, pbytes, p.nz);
     const C zc(HZ ? p.z + col * p.ldz : p.x, pbytes, p.nz), oc(p.out + col * p.ldo, pbytes, p.nz);
+    const C nc(STEP ? p.xn + col * p.ldn : p.out, pbytes, p.nz);
     // LDS cells (elements, buffer 0), all 16-byte aligned: my group (threads
     // past the block's rows read row 0's and write nothing), my halo group.
     // Cells left of a row and from nx on hold the points at its other end
@@ -745,9 +753,10 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
         T *pl = lds + ((z - zs) & 1) * psz;
         const F xv = xn;
         // consumed after the x / y sums of this plane (z: of output plane z - 6)
-        F vv, zz;
+        F vv, zz, xo;
         if (HV) vv = vc.load(z, off);
         if (HZ) zz = zc.load(max(z - kR, zs), off);
+        if (STEP) xo = x.load(max(z - kR, zs), off);
         if constexpr (PART) {
             if (act && !last) *reinterpret_cast<F *>(pl + own) = xv;
             // element by element: cells of any alignment, the last group's
@@ -770,7 +779,10 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
             hn = x.load(zn, hoff);
         }
         __syncthreads();
-        F xy = p.w0 * xv;
+        // smallest weights first, the centre's (the largest) last: the x and y
+        // sums then round at their own size (all terms on top of w0 x gave the
+        // FP32 Hamiltonian 1.5 times stencil_tiled's error)
+        F sx, sy;
         {
             T line[(2 * HG + 1) * V];
 #pragma unroll
@@ -782,20 +794,24 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
                 for (int e = 0; e < V; e++) line[q * V + e] = w[e];
             }
 #pragma unroll
-            for (int s = 1; s <= kR; s++)
+            for (int e = 0; e < V; e++) {
+                sx[e] = p.wx[kR] * (line[HG * V + e - kR] + line[HG * V + e + kR]);
 #pragma unroll
-                for (int e = 0; e < V; e++)
-                    xy[e] += p.wx[s] * (line[HG * V + e - s] + line[HG * V + e + s]);
+                for (int s = kR - 1; s >= 1; s--)
+                    sx[e] += p.wx[s] * (line[HG * V + e - s] + line[HG * V + e + s]);
+            }
         }
         // the y rows in two halves (all at once would hold 24 registers more)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 1; s <= kR; s++) {
+        for (int s = kR; s >= 1; s--) {
             const F a = *reinterpret_cast<const F *>(pl + own - s * rs);
             const F b = *reinterpret_cast<const F *>(pl + own + s * rs);
-            xy += p.wy[s] * (a + b);
-            if (s == kR / 2) __builtin_amdgcn_sched_barrier(0);
+            if (s == kR) sy = p.wy[s] * (a + b);
+            else sy += p.wy[s] * (a + b);
+            if (s == kR / 2 + 1) __builtin_amdgcn_sched_barrier(0);
         }
+        F xy = (sx + sy) + p.w0 * xv;
         if (HV) xy += p.bdiag * (vv * xv);
         F done;
 #pragma unroll
@@ -813,18 +829,24 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
         const bool out = z - kR >= zs;
         oc.store(max(z - kR, zs), out ? off_w : kNoRow, done);
         if (PART) oc.store_part(max(z - kR, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, done, rem);
+        if (STEP) {
+            xo += p.omega * done;
+            nc.store(max(z - kR, zs), out ? off_w : kNoRow, xo);
+            if (PART) nc.store_part(max(z - kR, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, xo, rem);
+        }
     }
     // planes ze .. ze + 5 finish outputs ze - 6 .. ze - 1 (those from zs on),
     // three at a time
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         constexpr int H = kR / 2;
-        F pos[H], zt[H];
+        F pos[H], zt[H], xt[H];
 #pragma unroll
         for (int j = 0; j < H; j++) {
             pos[j] = xplane(ze + h * H + j, off);
             const int zo = ze - kR + h * H + j;
             if (HZ) zt[j] = zc.load(max(zo, zs), off);
+            if (STEP) xt[j] = x.load(max(zo, zs), off);
         }
 #pragma unroll
         for (int j = 0; j < H; j++) {
@@ -837,6 +859,12 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
             const bool out = zo >= zs;
             oc.store(max(zo, zs), out ? off_w : kNoRow, o);
             if (PART) oc.store_part(max(zo, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, o, rem);
+            if (STEP) {
+                xt[j] += p.omega * o;
+                nc.store(max(zo, zs), out ? off_w : kNoRow, xt[j]);
+                if (PART)
+                    nc.store_part(max(zo, zs), out ? off_2 : kNoRow, out ? off_1 : kNoRow, xt[j], rem);
+            }
         }
     }
 }
@@ -846,7 +874,7 @@ __global__ __launch_bounds__(1024) void stencil_march(StencilParams<T> p, int gx
 // from L2 with all loads of a thread in flight at once.  What bounds it is one
 // memory latency plus the launch, where the marching forms pay a latency per
 // plane; the 13-fold reads stay in L2 / L1 as long as the block does.
-template <typename T, bool HV, bool HZ>
+template <typename T, bool HV, bool HZ, bool STEP>
 __global__ __launch_bounds__(256) void stencil_near(StencilParams<T> p, int gx)
 {
     using C = Column<T>;
@@ -916,13 +944,17 @@ __global__ __launch_bounds__(256) void stencil_near(StencilParams<T> p, int gx)
         o[e] = p.s1 * res;
         if (HZ) o[e] += p.s2 * zz[e];
     }
-    if (skip == 0) {
-        oc.store(z, off, o);
-    } else {
+    auto put = [&](const C &to, const F &v) {
+        if (skip == 0) {
+            to.store(z, off, v);
+        } else {
 #pragma unroll
-        for (int e = 1; e < V; e++)
-            if (e >= skip) oc.store1(z, act ? off + e * (int)sizeof(T) : kNoRow, o[e]);
-    }
+            for (int e = 1; e < V; e++)
+                if (e >= skip) to.store1(z, act ? off + e * (int)sizeof(T) : kNoRow, v[e]);
+        }
+    };
+    put(oc, o);
+    if (STEP) put(C(p.xn + col * p.ldn, pb, p.nz), c + p.omega * o);
 }
 
 template <typename T, int TX, int TY, int RY, int NS>
@@ -992,10 +1024,13 @@ void launch_near(sgpu_context *ctx, const StencilParams<T> &p, int ncol)
     const dim3 grid((ctx->ny * gx + 255) / 256, ctx->nz, ncol);
     const bool hv = p.bdiag != T(0), hz = p.z != nullptr;
     auto go = [&](auto kern) { kern<<<grid, 256, 0, ctx->stream>>>(p, gx); };
-    if (hv && hz) go(stencil_near<T, true, true>);
-    else if (hv) go(stencil_near<T, true, false>);
-    else if (hz) go(stencil_near<T, false, true>);
-    else go(stencil_near<T, false, false>);
+    if constexpr (sizeof(T) == 8) {
+        if (p.xn) return go(stencil_near<T, false, true, true>);
+    }
+    if (hv && hz) go(stencil_near<T, true, true, false>);
+    else if (hv) go(stencil_near<T, true, false, false>);
+    else if (hz) go(stencil_near<T, false, true, false>);
+    else go(stencil_near<T, false, false, false>);
 }
 
 template <typename T>
@@ -1007,17 +1042,18 @@ void launch_march(sgpu_context *ctx, const StencilParams<T> &p, int ncol, const 
     const dim3 grid((ctx->ny + ty - 1) / ty, ncol, (ctx->nz + zchunk - 1) / zchunk);
     const bool hv = p.bdiag != T(0), hz = p.z != nullptr;
     auto go = [&](auto kern) { kern<<<grid, nt, shm, ctx->stream>>>(p, gx, ty, zchunk); };
-    if (ctx->nx % March<T>::V) {
-        if (hv && hz) go(stencil_march<T, true, true, true>);
-        else if (hv) go(stencil_march<T, true, false, true>);
-        else if (hz) go(stencil_march<T, false, true, true>);
-        else go(stencil_march<T, false, false, true>);
-    } else {
-        if (hv && hz) go(stencil_march<T, true, true, false>);
-        else if (hv) go(stencil_march<T, true, false, false>);
-        else if (hz) go(stencil_march<T, false, true, false>);
-        else go(stencil_march<T, false, false, false>);
-    }
+    auto with_part = [&](auto part) {
+        constexpr bool PART = decltype(part)::value;
+        if constexpr (sizeof(T) == 8) {
+            if (p.xn) return go(stencil_march<T, false, true, PART, true>);
+        }
+        if (hv && hz) go(stencil_march<T, true, true, PART, false>);
+        else if (hv) go(stencil_march<T, true, false, PART, false>);
+        else if (hz) go(stencil_march<T, false, true, PART, false>);
+        else go(stencil_march<T, false, false, PART, false>);
+    };
+    if (ctx->nx % March<T>::V) with_part(std::true_type{});
+    else with_part(std::false_type{});
 }
 
 // Largest block stencil_near takes: below it one latency beats the marching
@@ -1170,9 +1206,9 @@ int tune_tile(sgpu_context *ctx, StencilParams<T> p, int ncol, int *best_cfg)
 }
 
 template <typename T>
-int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, const T *v,
-                 const T *x, long ldx, T *out, long ldo, const T *z, long ldz, double s1,
-                 double s2, bool allow_tiled, bool may_tune)
+StencilParams<T> stencil_params(const sgpu_context *ctx, double a, double bdiag, double c, const T *v,
+                                const T *x, long ldx, T *out, long ldo, const T *z, long ldz,
+                                double s1, double s2)
 {
     StencilParams<T> p;
     p.x = x; p.out = out; p.z = z; p.v = v;
@@ -1188,6 +1224,18 @@ int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, 
     p.bdiag = (v && std::fabs(bdiag) >= 1e-14) ? (T)bdiag : T(0);
     p.s1 = (T)s1;
     p.s2 = (T)s2;
+    p.xn = nullptr;
+    p.ldn = 0;
+    p.omega = T(0);
+    return p;
+}
+
+template <typename T>
+int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, const T *v,
+                 const T *x, long ldx, T *out, long ldo, const T *z, long ldz, double s1,
+                 double s2, bool allow_tiled, bool may_tune, bool tiles_only)
+{
+    const StencilParams<T> p = stencil_params<T>(ctx, a, bdiag, c, v, x, ldx, out, ldo, z, ldz, s1, s2);
     if (p.bdiag != T(0) && !v) {
         sgpu_set_error("stencil: diagonal requested without Veff");
         return SGPU_ERR_STATE;
@@ -1199,7 +1247,7 @@ int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, 
     }
     if (allow_tiled && ctx->fdn == kR) {
         int cfg = ctx->stencil_cfg;
-        if (launch_vec<T>(ctx, p, ncol, cfg)) {
+        if (!tiles_only && launch_vec<T>(ctx, p, ncol, cfg)) {
             SGPU_HIP(hipGetLastError());
             return SGPU_OK;
         }
@@ -1207,13 +1255,15 @@ int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, 
         if (cfg < 0) {
             const auto key = std::make_pair((int)sizeof(T), ncol);
             auto it = ctx->tile_choice.find(key);
-            if (it == ctx->tile_choice.end() && !may_tune) {
-                cfg = 0;
-            } else if (it == ctx->tile_choice.end()) {
+            if (it != ctx->tile_choice.end() && it->second < 20) {
+                cfg = it->second;
+            } else if (!may_tune || tiles_only) {
+                // few columns: thin z-chunks, or most CUs have no block (52^3 x 1
+                // FP64 about 20 -> 10 us)
+                cfg = ncol < 16 ? 10 : 0;
+            } else {
                 SGPU_CHECK(tune_tile<T>(ctx, p, ncol, &cfg));
                 ctx->tile_choice[key] = cfg;
-            } else {
-                cfg = it->second;
             }
         }
         launch_cfg<T>(ctx, p, ncol, cfg);
@@ -1238,15 +1288,31 @@ int launch_typed(sgpu_context *ctx, int ncol, double a, double bdiag, double c, 
 
 int sgpu_launch_stencil(sgpu_context *ctx, int dtype, int ncol, double a, double bdiag, double c,
                         const void *v, const void *x, long ldx, void *out, long ldo, const void *z,
-                        long ldz, double s1, double s2, bool allow_tiled, bool may_tune)
+                        long ldz, double s1, double s2, bool allow_tiled, bool may_tune,
+                        bool tiles_only)
 {
     if (dtype == SGPU_F64)
         return launch_typed<double>(ctx, ncol, a, bdiag, c, (const double *)v, (const double *)x,
                                     ldx, (double *)out, ldo, (const double *)z, ldz, s1, s2,
-                                    allow_tiled, may_tune);
+                                    allow_tiled, may_tune, tiles_only);
     return launch_typed<float>(ctx, ncol, a, bdiag, c, (const float *)v, (const float *)x, ldx,
                                (float *)out, ldo, (const float *)z, ldz, s1, s2, allow_tiled,
-                               may_tune);
+                               may_tune, tiles_only);
+}
+
+int sgpu_launch_aar_step(sgpu_context *ctx, double c, const double *x, const double *b, double *f,
+                         double *xn, double jac, double omega, bool *done)
+{
+    *done = false;
+    if (ctx->fdn != kR) return SGPU_OK;
+    StencilParams<double> p = stencil_params<double>(ctx, 1.0, 0.0, c, nullptr, x, ctx->ld, f, ctx->ld,
+                                                     b, ctx->ld, jac, jac);
+    p.xn = xn;
+    p.ldn = ctx->ld;
+    p.omega = omega;
+    *done = launch_vec<double>(ctx, p, 1, ctx->stencil_cfg);
+    SGPU_HIP(hipGetLastError());
+    return SGPU_OK;
 }
 
 extern "C" int sgpu_stencil_tile(const sgpu_context *ctx, int dtype, int ncol, int *tx, int *ty,
@@ -1304,10 +1370,10 @@ extern "C" int sgpu_stencil_kernel(const sgpu_context *ctx, int dtype, int ncol,
     if (tx == 0)
         name[0] = 0;
     else if (cfg == 20)
-        snprintf(name, len, "stencil_march<%s,true,true,%s>", t,
+        snprintf(name, len, "stencil_march<%s,true,true,%s,false>", t,
                  ctx->nx % (dtype == SGPU_F64 ? 2 : 4) ? "true" : "false");
     else if (cfg == 21)
-        snprintf(name, len, "stencil_near<%s,true,true>", t);
+        snprintf(name, len, "stencil_near<%s,true,true,false>", t);
     else if ((cfg == 13 || cfg == 14) && dtype != SGPU_F64 && ctx->nx == tx)
         snprintf(name, len, "stencil_rows<%d,%d,%d>", tx, ty, ry);
     else if ((cfg == 5 || cfg == 6) && dtype != SGPU_F64)

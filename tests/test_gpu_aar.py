@@ -52,3 +52,27 @@ def test_aar_deterministic(gpu):
         x2, it2, _, _ = ctx.AAR(np.zeros(g.nd), rhs, tol=1e-8, max_iter=500)
     assert it1 == it2
     assert np.array_equal(x1, x2)
+
+
+@pytest.mark.parametrize("n,m,p,c", [(20, 7, 6, 0.0), (21, 3, 2, 0.0), (24, 8, 5, -1.0), (33, 2, 7, 0.0),
+                                     (17, 5, 1, -0.5), (14, 7, 6, 0.0)])
+def test_aar_histories(gpu, oracle_mod, n, m, p, c):
+    """Ring histories of every kind against the oracle: more Richardson steps
+    between two Anderson steps than the history holds (p > m), fewer, and
+    Anderson at every step (p = 1, all differences from x), shifted operators,
+    the one-launch step (n >= 20), its remainders (odd n) and the general path
+    (n = 17, 14).  Both solve to 1e-10 of the residual; the solutions then agree
+    to that times the operator's condition, below 1e4 here."""
+    from sparc_amd.workloads import poisson_workload
+    g, rhs = poisson_workload(n=n, h=0.4, n_charges=6, seed=n)
+    o = oracle_mod.Oracle(g)
+    xo, it_o, rr_o = o.aar(np.zeros(g.nd), rhs, c=c, m=m, p=p, tol=1e-10, max_iter=3000)
+    with gpu.Context(g) as ctx:
+        x, it, rr, conv = ctx.AAR(np.zeros(g.nd), rhs, c=c, m=m, p=p, tol=1e-10, max_iter=3000)
+    assert conv and rr <= 1e-10
+    assert abs(it - it_o) <= max(12, it_o // 5)
+    if c == 0.0:
+        x, xo = x - x.mean(), xo - xo.mean()
+    assert rel_err(x, xo) < 1e-6
+    r = rhs + o.lap_vec_mult(x, c)[:, 0]
+    assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(rhs) + 1e-13 * np.linalg.norm(x) * 60.0
