@@ -7,20 +7,19 @@
 // dense Phi_b (kBP points x np_b projector columns of every atom touching
 // it).  The apply is then three launches over bricks x column blocks:
 //
-//  1. nlb_project_rs: part[brick rows][cols] = Phi_b' X_b on 16x16x4 MFMA,
-//     64 (FP32) / 32 (FP64) columns per block, X streamed from memory
-//     straight into the MFMA operands (16-byte loads of four consecutive
-//     points per lane), each wavefront taking a quarter of the brick's
-//     points, the four partial tiles summed in a fixed order through LDS.
+//  1. nlb_chain (projection only): part[brick rows][cols] = Phi_b' X_b on
+//     16x16x4 MFMA, 128 columns per block, 16 per wavefront.
 //  2. nlb_reduce: alpha_s[r][c] = scale dV Gamma_r sum over the brick rows of
 //     projector r (fixed order: deterministic, no atomics).
-//  3. nlb_apply_rs: out_b += Phi_b beta_b on 16x16x4 MFMA with beta_b
-//     (np_b x NC) gathered from alpha_s into LDS, computed with points as
-//     MFMA rows so that each lane's results are four consecutive points of
-//     one column (one 16-byte read-add-write).  Optionally it also forms the
-//     next Chebyshev step's partials from the updated values (the brick
-//     chain, SPARC_AMD_NL_CHAIN_BRICK=1).
+//  3. nlb_chain: out_b += Phi_b beta_b, computed with points as MFMA rows so
+//     that each lane's results are four consecutive points of one column (one
+//     16-byte read-add-write); in a Chebyshev chain the same pass forms the
+//     next step's partials from the updated values (SPARC_AMD_NL_CHAIN_BRICK=0
+//     keeps them apart), so 1. runs once per filter.
 //
+// Bricks of more than 112 rows take nlb_project_rs (X streamed straight into
+// the MFMA operands, the four wavefronts splitting the brick's points) and
+// nlb_apply_rs (beta in LDS).
 // The LDS-staged forms (nlb_project, 16 columns per block; the transposed
 // nlb_apply, 32 columns) stay selectable with SPARC_AMD_NLB=lds.  On the
 // 96^3 x 512 FP32 operator case: 1.04 -> 0.74 ms (projection) and
@@ -33,6 +32,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
+#include <type_traits>
 
 #include "sgpu_internal.h"
 
@@ -521,22 +521,16 @@ __global__ __launch_bounds__(256) void nlb_apply(T *__restrict__ out, long ldo, 
 // covering 16 columns' 64-byte (128-byte) segments of the row, and the A
 // operand (Phi_b column-major, points contiguous) is a coalesced load shared
 // by the NC / 16 column tiles.
-// With PROJ the updated values, still in registers, are also the B operands
-// of the projection Phi_b' out (point 4 lk + u in MFMA u, as in
-// nlb_project_rs): the pass writes the partials of out for the next
-// application of a Chebyshev chain into part_next, all RTM row tiles
-// accumulated at once (np <= 16 RTM), the four waves' tiles summed in a fixed
-// order.  Every lane's loads of a row step are issued before its MFMAs.
-template <typename T, int NC, int RTM, bool PROJ>
+// Every lane's loads of a row step are issued before its MFMAs.  Taken by bricks
+// of more rows than nlb_chain holds.
+template <typename T, int NC>
 __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ldo, int ncol, int nx,
                                                     int ny, int nz, const int *__restrict__ brick_org,
                                                     const int *__restrict__ brick_np,
                                                     const long *__restrict__ brick_row,
                                                     const int *__restrict__ row_alpha,
-                                                    const T *__restrict__ phi,
                                                     const T *__restrict__ phic,
-                                                    const T *__restrict__ alpha_s,
-                                                    T *__restrict__ part_next)
+                                                    const T *__restrict__ alpha_s)
 {
     using M = Mfma<T>;
     using V = typename Vec16<T>::type;
@@ -547,7 +541,6 @@ __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ld
     constexpr int PW = kBP / kWaves;          // points per wave
     extern __shared__ unsigned char smem_raw[];
     T *beta = reinterpret_cast<T *>(smem_raw);  // np x LDB
-    __shared__ typename M::acc red[PROJ ? RTM * NCT : 1][64];
     const int lid = xcd_remap(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int b = lid / gridDim.x;
     const int col0 = (lid % gridDim.x) * NC;
@@ -577,7 +570,6 @@ __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ld
     }
     __syncthreads();
     const T *pc = phic + row0 * kBP;
-    const T *ph = phi + row0 * kBP;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, lk = lane >> 4;
     // MFMA row li of a tile holds point prow (the D layout puts row i of
@@ -590,18 +582,6 @@ __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ld
         const int col = col0 + ct * 16 + li;
         cok[ct] = col < ncol;
         coff[ct] = cok[ct] ? (long)col * ldo : 0L;
-    }
-    typename M::acc pacc[PROJ ? RTM : 1][NCT];
-    if constexpr (PROJ) {
-#pragma unroll
-        for (int rt = 0; rt < RTM; rt++)
-#pragma unroll
-            for (int ct = 0; ct < NCT; ct++) pacc[rt][ct] = typename M::acc{0, 0, 0, 0};
-    }
-    int jr[PROJ ? RTM : 1];
-    if constexpr (PROJ) {
-#pragma unroll
-        for (int rt = 0; rt < RTM; rt++) jr[rt] = min(rt * 16 + li, np - 1);
     }
 #pragma unroll 1
     for (int t = 0; t < PW / 16; t++) {
@@ -673,56 +653,248 @@ __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ld
                     if (pts[r] >= 0) out[coff[ct] + pts[r]] = y[ct][r];
             }
         }
-        if constexpr (PROJ) {
-            // points outside the grid or columns past ncol contribute zero
+    }
+}
+
+// out_b += Phi_b beta_b for 128 columns, and (PROJ) the partials Phi_b' out of
+// the result for the next application of a Chebyshev chain, in one pass: out
+// is read and written once and the next projection does not read it again.
+// Each of the eight waves owns 16 columns and walks the brick's 512 points in
+// 16-point x-rows; its beta operands (np / 4 per lane) and the projection's
+// accumulators (np / 16 tiles) stay in registers for the whole brick, so the
+// waves share nothing but Phi_b, which is staged once for all 128 columns, a
+// chunk of points at a time ([row][point], double-buffered, one barrier per
+// chunk), and serves both products: the apply reads it as A (point, j) with
+// nlb_apply_rs's row order, so that a lane's four results are the points
+// 4 lk .. 4 lk + 3 of its column, and the projection as A (j, point 4 lk + u),
+// for which those four values are the B operands.  A chunk's out values are
+// loaded while the chunk before is multiplied.
+// What bounds it: HBM (out once in, once out: 3.6 GB at 96^3 x 512 FP32, at
+// 3.2 TB/s), with the matrix cores busy for half of it.  Per application there
+// 1.14 ms (FP64 2.46) against 1.16 + 0.75 ms (2.36 + 1.9) for nlb_apply_rs and
+// nlb_project_rs, whose 64-column blocks read Phi from L2 in every wave and the
+// block three times; the two apart in this form 1.01 + 0.57 (2.12 + 1.37).
+// A switch on the tiles per brick keeps the products and operand loads free of
+// conditions (1.25 ms with them).
+// VEC: a lane's four points lie in the grid together (nx a multiple of 4).
+// Without APPLY it is the projection alone (out only read), with the same sums.
+template <typename T>
+struct Chain {
+    static constexpr int NW = 8, NC = 16 * NW;
+    static constexpr int CH = sizeof(T) == 4 ? 64 : 32;  // points per chunk
+    static constexpr int LDP = CH + 16 / (int)sizeof(T) * 2;
+    static constexpr int RTM = 7;                        // most 16-row tiles per brick
+    static size_t shmem(int max_np) { return (size_t)2 * ((max_np + 15) / 16 * 16) * LDP * sizeof(T); }
+};
+
+// RT: 16-row tiles of this brick.
+template <typename T, bool VEC, bool APPLY, bool PROJ, int RT>
+__device__ __forceinline__ void nlb_chain_brick(
+    T *ph, T *out, long ldo, int ncol, int nx, int ny, int nz, int b, int cb, int np,
+    const int *__restrict__ brick_org, const long *__restrict__ brick_row,
+    const int *__restrict__ row_alpha, const T *__restrict__ phic, const T *__restrict__ alpha_s,
+    T *__restrict__ part_next)
+{
+    using M = Mfma<T>;
+    using K = Chain<T>;
+    using acc_t = typename M::acc;
+    using V = typename Vec16<T>::type;
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    constexpr int VW = 16 / sizeof(T), NV = 4 / VW, SZ = sizeof(T);
+    constexpr int CH = K::CH, LDP = K::LDP, NS = CH / 16;  // NS x-rows per chunk
+    constexpr int BUF = 16 * RT * LDP;
+    constexpr int kOff = 0x7ffffff0;  // past every resource: reads zero, stores nothing
+    const int x0 = brick_org[3 * b], y0 = brick_org[3 * b + 1], z0 = brick_org[3 * b + 2];
+    const long row0 = brick_row[b];
+    const T *pc = phic + row0 * kBP;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int prow = sizeof(T) == 4 ? li : 4 * (li & 3) + (li >> 2);
+    const int c0 = cb * K::NC + wave * 16;
+    const int nc = max(0, min(16, ncol - c0));
+    // my wave's columns as one buffer resource
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(out + (long)min(c0, ncol - 1) * ldo), 0, (int)(nc * ldo * SZ), 0x00020000);
+    const bool cok = li < nc;
+    // lane part of the offset of my four points (element e for !VEC)
+    const int xl = x0 + 4 * lk;
+    const int vo = cok && xl < nx ? (int)((li * ldo + xl) * SZ) : kOff;
+    auto row_off = [&](int step) {  // byte offset of x-row `step` of the brick, -1: outside
+        const int y = y0 + step % kBY, z = z0 + step / kBY;
+        return y < ny && z < nz ? (z * ny + y) * nx * SZ : -1;
+    };
+    auto load4 = [&](int step, T (&v)[4]) {
+        const int ro = row_off(step);
+        if constexpr (VEC) {
+            const int o = ro < 0 ? kOff : vo;
 #pragma unroll
-            for (int ct = 0; ct < NCT; ct++)
+            for (int q = 0; q < NV; q++) {
+                const V w = __builtin_bit_cast(
+                    V, __builtin_amdgcn_raw_buffer_load_b128(rc, o + q * 16, ro < 0 ? 0 : ro, 0));
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (pts[r] < 0 || !cok[ct]) y[ct][r] = T(0);
+                for (int e = 0; e < VW; e++) v[q * VW + e] = w[e];
+            }
+        } else {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                T aph[RTM];
-#pragma unroll
-                for (int rt = 0; rt < RTM; rt++) aph[rt] = ph[(long)(q0 + 4 * lk + u) * np + jr[rt]];
-#pragma unroll
-                for (int rt = 0; rt < RTM; rt++) {
-                    if (rt * 16 < np) {
-#pragma unroll
-                        for (int ct = 0; ct < NCT; ct++)
-                            pacc[rt][ct] = M::run(aph[rt], y[ct][u], pacc[rt][ct]);
-                    }
-                }
+            for (int e = 0; e < 4; e++) {
+                const int o = ro < 0 || xl + e >= nx ? kOff : vo + e * SZ;
+                if constexpr (SZ == 4)
+                    v[e] = __builtin_bit_cast(
+                        T, __builtin_amdgcn_raw_buffer_load_b32(rc, o, ro < 0 ? 0 : ro, 0));
+                else
+                    v[e] = __builtin_bit_cast(
+                        T, __builtin_amdgcn_raw_buffer_load_b64(rc, o, ro < 0 ? 0 : ro, 0));
             }
         }
+    };
+    // (stores take the row in the vector offset, see stencil.hip's Column)
+    auto store4 = [&](int step, const T (&v)[4]) {
+        const int ro = row_off(step);
+        if constexpr (VEC) {
+            const unsigned o = ro < 0 ? (unsigned)kOff : (unsigned)vo + (unsigned)ro;
+#pragma unroll
+            for (int q = 0; q < NV; q++) {
+                V w;
+#pragma unroll
+                for (int e = 0; e < VW; e++) w[e] = v[q * VW + e];
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, w), rc, o + q * 16, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned o =
+                    ro < 0 || xl + e >= nx ? (unsigned)kOff : (unsigned)vo + (unsigned)ro + e * SZ;
+                if constexpr (SZ == 4)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[e]), rc, o, 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v[e]), rc, o, 0, 0);
+            }
+        }
+    };
+
+    // the first chunk's out values, then beta (B (j, col), zero for absent columns)
+    T ov[NS][4];
+#pragma unroll
+    for (int t = 0; t < NS; t++) load4(t, ov[t]);
+    T beta[APPLY ? 4 * RT : 1];
+#pragma unroll
+    for (int s = 0; s < (APPLY ? 4 * RT : 0); s++) {
+        const int j = 4 * s + lk;
+        const int r = j < np ? row_alpha[row0 + j] : -1;
+        const bool ok = r >= 0 && cok;
+        const T v = alpha_s[ok ? (long)r * ncol + c0 + li : 0L];
+        beta[s] = ok ? v : T(0);
+    }
+    acc_t pacc[PROJ ? RT : 1];
+#pragma unroll
+    for (int rt = 0; rt < (PROJ ? RT : 1); rt++) pacc[rt] = acc_t{0, 0, 0, 0};
+    // Phi staging: 16-byte pieces f of the chunk's np rows
+    constexpr int PV = CH / VW;                      // pieces per row
+    constexpr int kS = (16 * RT * PV + 511) / 512;  // per thread
+    V st[kS];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int q = 0; q < kS; q++) {
+            // rows np .. 16 RT are staged as zeros, so no tile is cut short
+            const int f = threadIdx.x + 512 * q, j = f / PV;
+            const V w = *reinterpret_cast<const V *>(pc + (long)min(j, np - 1) * kBP + c * CH + (f % PV) * VW);
+            st[q] = j < np ? w : V(T(0));
+        }
+    };
+    auto put = [&](int c) {
+        T *dst = ph + (c & 1) * BUF;
+#pragma unroll
+        for (int q = 0; q < kS; q++) {
+            const int f = threadIdx.x + 512 * q;
+            if (f < 16 * RT * PV) *reinterpret_cast<V *>(dst + (f / PV) * LDP + (f % PV) * VW) = st[q];
+        }
+    };
+    fetch(0);
+    put(0);
+    constexpr int NCH = kBP / CH;
+#pragma unroll 1
+    for (int c = 0; c < NCH; c++) {
+        if (c + 1 < NCH) fetch(c + 1);
+        __syncthreads();  // chunk c is staged, chunk c - 1 is read
+        const T *pp = ph + (c & 1) * BUF;
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+            T y[4];
+            if constexpr (APPLY) {
+                acc_t acc = acc_t{0, 0, 0, 0};
+                const T *pa = pp + lk * LDP + t * 16 + prow;
+#pragma unroll
+                for (int s = 0; s < 4 * RT; s++) acc = M::run(pa[4 * s * LDP], beta[s], acc);
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] = ov[t][e] + acc[e];
+                store4(c * NS + t, y);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] = ov[t][e];
+            }
+            if (c + 1 < NCH) load4((c + 1) * NS + t, ov[t]);
+            if constexpr (PROJ) {
+                // points and columns outside contribute zero
+                const bool in = row_off(c * NS + t) >= 0 && cok;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (!in || (VEC ? xl : xl + e) >= nx) y[e] = T(0);
+                const T *pj = pp + li * LDP + t * 16 + 4 * lk;
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) {
+                    T a[4];
+#pragma unroll
+                    for (int q = 0; q < NV; q++) {
+                        const V w = *reinterpret_cast<const V *>(pj + 16 * rt * LDP + q * VW);
+#pragma unroll
+                        for (int e = 0; e < VW; e++) a[q * VW + e] = w[e];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) pacc[rt] = M::run(a[u], y[u], pacc[rt]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (the steps' operands in turn, not all at once)
+        }
+        if (c + 1 < NCH) put(c + 1);
     }
     if constexpr (PROJ) {
-        for (int w = kWaves - 1; w >= 1; w--) {
-            if (wave == w)
 #pragma unroll
-                for (int rt = 0; rt < RTM; rt++)
+        for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-                    for (int ct = 0; ct < NCT; ct++) red[rt * NCT + ct][lane] = pacc[rt][ct];
-            __syncthreads();
-            if (wave == w - 1)
-#pragma unroll
-                for (int rt = 0; rt < RTM; rt++)
-#pragma unroll
-                    for (int ct = 0; ct < NCT; ct++) pacc[rt][ct] += red[rt * NCT + ct][lane];
-            __syncthreads();
-        }
-        if (wave == 0) {
-#pragma unroll
-            for (int rt = 0; rt < RTM; rt++)
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int j = rt * 16 + M::drow(lk, r);
-                        const int col = col0 + ct * 16 + li;
-                        if (j < np && col < ncol) part_next[(row0 + j) * ncol + col] = pacc[rt][ct][r];
-                    }
-        }
+            for (int r = 0; r < 4; r++) {
+                const int j = rt * 16 + M::drow(lk, r);
+                if (j < np && cok) part_next[(row0 + j) * ncol + c0 + li] = pacc[rt][r];
+            }
+    }
+}
+
+template <typename T, bool VEC, bool APPLY, bool PROJ>
+__global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 2) void nlb_chain(
+    T *out, long ldo, int ncol, int nx, int ny, int nz, const int *__restrict__ brick_org,
+    const int *__restrict__ brick_np, const long *__restrict__ brick_row,
+    const int *__restrict__ row_alpha, const T *__restrict__ phic, const T *__restrict__ alpha_s,
+    T *__restrict__ part_next)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T *ph = reinterpret_cast<T *>(smem_raw);  // [2][16 RT][LDP]
+    const int lid = xcd_remap(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
+    const int b = lid / gridDim.x, cb = lid % gridDim.x;
+    const int np = brick_np[b];
+    auto go = [&](auto rt) {
+        nlb_chain_brick<T, VEC, APPLY, PROJ, decltype(rt)::value>(ph, out, ldo, ncol, nx, ny, nz, b, cb, np,
+                                                                  brick_org, brick_row, row_alpha, phic,
+                                                                  alpha_s, part_next);
+    };
+    switch ((np + 15) / 16) {
+        case 1: go(std::integral_constant<int, 1>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 3: go(std::integral_constant<int, 3>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 5: go(std::integral_constant<int, 5>{}); break;
+        case 6: go(std::integral_constant<int, 6>{}); break;
+        default: go(std::integral_constant<int, 7>{}); break;
     }
 }
 
@@ -1205,14 +1377,42 @@ bool nlb_lds_kernels()
     return v;
 }
 
-// Rows of Phi_b the fused apply + projection accumulates at once.
-constexpr int kChainRTM = 7;
+// Whether nlb_chain takes the layout: its register tiles hold the bricks' rows
+// and 16 columns stay below 2^31 bytes.
+template <typename T>
+bool nlb_chain_fits(const sgpu_context *ctx, long ldo)
+{
+    return !nlb_lds_kernels() && ctx->nl.max_np <= 16 * Chain<T>::RTM &&
+           16 * ldo * (long)sizeof(T) < 0x7ffffff0L;
+}
+
+template <typename T, bool APPLY, bool PROJ>
+int launch_nlb_chain(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phic, const T *alpha_s,
+                     T *part_next)
+{
+    using K = Chain<T>;
+    const sgpu_nonlocal &nl = ctx->nl;
+    const size_t shm = K::shmem(nl.max_np);
+    const dim3 grid((ncol + K::NC - 1) / K::NC, nl.n_bricks);
+    auto go = [&](auto kern) {
+        if (shm > 32 * 1024)
+            SGPU_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+        kern<<<grid, 512, shm, ctx->stream>>>(out, ldo, ncol, ctx->nx, ctx->ny, ctx->nz,
+                                              nl.brick_org, nl.brick_np, nl.brick_row, nl.row_alpha,
+                                              phic, alpha_s, part_next);
+        return SGPU_OK;
+    };
+    const bool vec = ctx->nx % 4 == 0 && ldo % (16 / (long)sizeof(T)) == 0 &&
+                     (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    return vec ? go(nlb_chain<T, true, APPLY, PROJ>) : go(nlb_chain<T, false, APPLY, PROJ>);
+}
 
 // out += Phi_b beta_b (beta_b gathered from alpha_s); with part_next also the
 // partials Phi_b' out of the result.
 template <typename T>
-int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi, const T *phic,
-                     const T *alpha_s, T *part_next)
+int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phic, const T *alpha_s,
+                     T *part_next)
 {
     const sgpu_nonlocal &nl = ctx->nl;
     if (nlb_lds_kernels() && !part_next) {
@@ -1228,6 +1428,11 @@ int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi
             nl.row_alpha, phic, alpha_s);
         return SGPU_OK;
     }
+    if (nlb_chain_fits<T>(ctx, ldo)) {
+        if (part_next)
+            return launch_nlb_chain<T, true, true>(ctx, ncol, out, ldo, phic, alpha_s, part_next);
+        return launch_nlb_chain<T, true, false>(ctx, ncol, out, ldo, phic, alpha_s, nullptr);
+    }
     constexpr int NC = Mfma<T>::NCB, LDB = NC + 64 / (int)sizeof(T);
     const size_t shmem = (size_t)nl.max_np * LDB * sizeof(T);
     if (shmem > 96 * 1024) {
@@ -1242,33 +1447,28 @@ int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
         kern<<<grid, 256, shmem, ctx->stream>>>(out, ldo, ncol, ctx->nx, ctx->ny, ctx->nz,
                                                 nl.brick_org, nl.brick_np, nl.brick_row,
-                                                nl.row_alpha, phi, phic, alpha_s, part_next);
+                                                nl.row_alpha, phic, alpha_s);
         return SGPU_OK;
     };
-    if (part_next) {
-        if (nl.max_np > 16 * kChainRTM) {
-            sgpu_set_error("nonlocal: fused apply + projection limited to %d rows per brick",
-                           16 * kChainRTM);
-            return SGPU_ERR_ARG;
-        }
-        return go(nlb_apply_rs<T, NC, kChainRTM, true>);
-    }
-    return go(nlb_apply_rs<T, NC, 1, false>);
+    return go(nlb_apply_rs<T, NC>);
 }
 
 // part = Phi_b' X for every brick: nlb_project_rs with 64 (FP32) / 32 (FP64)
 // columns per block, 16-byte loads where the grid and X allow them.
 template <typename T>
-void launch_nlb_project(sgpu_context *ctx, int ncol, const T *x, long ldx, const T *phi, T *part)
+int launch_nlb_project(sgpu_context *ctx, int ncol, const T *x, long ldx, const T *phi, const T *phic,
+                       T *part)
 {
     const sgpu_nonlocal &nl = ctx->nl;
     const hipStream_t stream = ctx->stream;
+    if (nlb_chain_fits<T>(ctx, ldx))
+        return launch_nlb_chain<T, false, true>(ctx, ncol, const_cast<T *>(x), ldx, phic, nullptr, part);
     if (nlb_lds_kernels()) {
         constexpr int NCP = Mfma<T>::NCP;
         nlb_project<T><<<dim3((ncol + NCP - 1) / NCP, nl.n_bricks), 256, 0, stream>>>(
             x, ldx, ncol, ctx->nx, ctx->ny, ctx->nz, nl.brick_org, nl.brick_np, nl.brick_row, phi,
             part);
-        return;
+        return SGPU_OK;
     }
     // 16-byte loads of four points: the points of a lane lie inside the grid
     // together when nx is a multiple of 4
@@ -1283,6 +1483,7 @@ void launch_nlb_project(sgpu_context *ctx, int ncol, const T *x, long ldx, const
         nlb_project_rs<T, NC, false><<<grid, 256, 0, stream>>>(
             x, ldx, ncol, ctx->nx, ctx->ny, ctx->nz, nl.brick_org, nl.brick_np, nl.brick_row, phi,
             part);
+    return SGPU_OK;
 }
 
 // The partials buffer: the caller's workspace when one is given (it must
@@ -1345,7 +1546,7 @@ int launch_vnl_typed(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, 
     T *alpha_s = part + part_elems;
     sgpu_tmark t;
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    launch_nlb_project<T>(ctx, ncol, x, ldx, phi, part);
+    SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     const long total = (long)nl.n_alpha * ncol;
@@ -1353,7 +1554,7 @@ int launch_vnl_typed(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, 
         part, ncol, nl.n_alpha, nl.arow_ptr, nl.arow_src, nl.gamma, scale * nl.dV, alpha_s);
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phi, phic, alpha_s, nullptr));
+    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s, nullptr));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
     return SGPU_OK;
@@ -1438,10 +1639,9 @@ int launch_vnl_chain_sphere(sgpu_context *ctx, int ncol, const T *x, long ldx, T
 
 // One application of a Chebyshev chain with the brick layout: the partials of
 // x are those the previous application left (have_part) or a projection of x;
-// with want_next the apply also forms the partials of out (nlb_apply_rs with
-// PROJ), so the next application skips its projection and the re-read of its
-// input.  Partials ping-pong between two buffers in nl.chain, alpha_s after
-// them.
+// with want_next the apply also forms the partials of out (nlb_chain), so the
+// next application skips its projection and the re-read of its input.  Partials
+// ping-pong between two buffers in nl.chain, alpha_s after them.
 template <typename T>
 int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, long ldo,
                            double scale, const T *phi, const T *phic, bool have_part,
@@ -1454,8 +1654,7 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
         sgpu_set_error("nonlocal: %d bricks exceed the launch limit", nl.n_bricks);
         return SGPU_ERR_ARG;
     }
-    const bool fuse = want_next && ctx->nl_chain_brick && !nlb_lds_kernels() &&
-                      nl.max_np <= 16 * kChainRTM;
+    const bool fuse = want_next && ctx->nl_chain_brick && nlb_chain_fits<T>(ctx, ldo);
     if (!fuse && !have_part)
         return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0);
     const size_t part_elems = (size_t)nl.n_rows * ncol;
@@ -1465,7 +1664,11 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
         return SGPU_ERR_STATE;
     }
     void *buf = nullptr;
-    SGPU_CHECK(chain_buffer(ctx, need, &buf));
+    if (chain_buffer(ctx, need, &buf) < 0) {
+        // no room for two sets of partials: the separate launches need one
+        (void)hipGetLastError();
+        return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0);
+    }
     if (!have_part) nl.chain_cur = 0;
     T *part = (T *)buf + (size_t)nl.chain_cur * part_elems;
     T *part_next = (T *)buf + (size_t)(nl.chain_cur ^ 1) * part_elems;
@@ -1473,7 +1676,7 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
     sgpu_tmark t;
     if (!have_part) {
         SGPU_CHECK(sgpu_tbegin(ctx, &t));
-        launch_nlb_project<T>(ctx, ncol, x, ldx, phi, part);
+        SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part));
         SGPU_HIP(hipGetLastError());
         SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     }
@@ -1482,7 +1685,7 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
         part, ncol, nl.n_alpha, nl.arow_ptr, nl.arow_src, nl.gamma, scale * nl.dV, alpha_s);
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phi, phic, alpha_s,
+    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s,
                                    fuse ? part_next : nullptr));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
@@ -1709,8 +1912,10 @@ int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scal
         }
         SGPU_CHECK(sgpu_scratch(ctx, (size_t)nl.n_rows * ncol * sizeof(T) + 256, &buf));
         T *part = (T *)buf;
-        launch_nlb_project<T>(ctx, ncol, x, ldx,
-                              sizeof(T) == 8 ? (const T *)nl.phi64 : (const T *)nl.phi32, part);
+        SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx,
+                                         sizeof(T) == 8 ? (const T *)nl.phi64 : (const T *)nl.phi32,
+                                         sizeof(T) == 8 ? (const T *)nl.phic64 : (const T *)nl.phic32,
+                                         part));
         SGPU_HIP(hipGetLastError());
         const long total = (long)nl.n_alpha * ncol;
         nlb_reduce<T><<<(unsigned)((total + 255) / 256), 256, 0, ctx->stream>>>(

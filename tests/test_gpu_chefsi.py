@@ -296,6 +296,37 @@ def test_filter_nonlocal_chain(gpu, oracle_mod, monkeypatch, mode, overlap, dtyp
     assert rel_err(out["1"], Yo) < (1e-11 if dtype == 0 else 1e-4)
 
 
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("n,sites,lmax,ncol", [
+    ((20, 18, 16), 1, 0, 1),      # two rows: one tile, one column
+    ((21, 17, 16), 4, 1, 129),    # 32 rows, x-rows ending inside a lane's four points, 129 columns
+    ((34, 20, 17), 5, 2, 16),     # 72 rows (five tiles, the last partly filled)
+    ((18, 16, 16), 7, 2, 128),    # 126 rows, above 112: the general kernels
+])
+def test_brick_chain_edges(gpu, oracle_mod, monkeypatch, n, sites, lmax, ncol, dtype):
+    """The brick layout's apply, projection and their fused form at the edges
+    of their tiles: the Chebyshev filter (fused) equal to the unfused one, and
+    both against the oracle.  Tolerances as in test_filter_nonlocal_chain."""
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "brick")
+    g, veff, nl, rng = small_case(n=n, n_sites=sites, rc=3.2, seed=61, lmax=lmax)
+    o = oracle_mod.Oracle(g, veff, nl)
+    a0, b, a = _bounds(o, g)
+    X = rng.uniform(-0.5, 0.5, (g.nd, ncol))
+    Yo, _ = o.chebyshev_filter(X, 4, a, b, a0)
+    out = {}
+    for fused in ("1", "0"):
+        monkeypatch.setenv("SPARC_AMD_NL_CHAIN_BRICK", fused)
+        with gpu.Context(g) as ctx:
+            ctx.set_veff(veff)
+            ctx.set_nonlocal(nl)
+            bx = ctx.block(ncol, dtype).upload(X)
+            by = ctx.block(ncol, dtype)
+            ctx.chebyshev_filter_dev(bx, by, 4, a, b, a0)
+            out[fused] = by.download()
+    assert np.array_equal(out["1"], out["0"])
+    assert rel_err(out["1"], Yo) < (1e-11 if dtype == 0 else 1e-4)
+
+
 @pytest.mark.parametrize("n,groups,threads", [(181, 32, 256), (300, 7, 256), (480, 32, 256),
                                               (480, 64, 512), (1000, 16, 256)])
 def test_generalized_eigensolve_cooperative_tridiagonal(gpu, monkeypatch, n, groups, threads):
