@@ -168,8 +168,8 @@ def nonlocal_dense(ctx, wl, rec, peak_key):
     chi, ns = int(wl.nloc.chi.size), wl.ncol
     out = {"layout": "bricks" if mode == 0 else "spheres", "stored_values": stored,
            "chi_values": chi}
-    names = {"nl_project": "nlb_project_rs" if mode == 0 else "nls_project",
-             "nl_apply": "nlb_apply_rs" if mode == 0 else "nls_apply / nls_apply_proj"}
+    names = {"nl_project": "nlb_chain" if mode == 0 else "nls_chain",
+             "nl_apply": "nlb_chain" if mode == 0 else "nls_chain"}
     for key in ("nl_project", "nl_apply"):
         tot, cnt = rec[key]
         if cnt:

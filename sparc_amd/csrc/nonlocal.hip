@@ -904,221 +904,38 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 2) void nlb_chain(
 // pseudopotentials, rc ~ 2 Bohr: ~500 points against ~6000 brick points) the
 // work follows the reference's gather / GEMM / scatter per atom instead:
 //
-//  1. nls_project: part[e][p][col] = sum_q Chi_e[q][p] X[col][pos_e[q]] on
-//     16x16x4 MFMA; the entry's points are staged in LDS 256 at a time
-//     (gathered, consecutive threads on consecutive points), the four waves
-//     split each chunk and their tiles are summed in a fixed order.
-//  2. nls_apply, one launch per colour: beta = scale dV Gamma sum over the
+//  1. nls_chain (projection only): part[e][p][col] = sum_q Chi_e[q][p] X[col][pos_e[q]].
+//  2. nls_chain, one launch per colour: beta = scale dV Gamma sum over the
 //     atom's images of part (fixed order), then out[col][pos_e[q]] +=
-//     sum_p Chi_e[q][p] beta[p][col] as the transposed tile (cols x points)
-//     so that every output register row is 16 consecutive points of one
-//     column.  Entries of one colour share no grid point, so the
-//     read-add-write needs no atomics and the result is deterministic.
-constexpr int kQC = 256;           // points staged per chunk (multiple of 64)
-constexpr int kQLD = kQC + 4;      // LDS stride of a staged column
-
-template <typename T>
-__global__ __launch_bounds__(256) void nls_project(const T *__restrict__ X, long ldx, int ncol,
-                                                   const int *__restrict__ ent_info,
-                                                   const long *__restrict__ ent_chi,
-                                                   const int *__restrict__ gpos,
-                                                   const T *__restrict__ chir, int max_np,
-                                                   T *__restrict__ part)
-{
-    using M = Mfma<T>;
-    constexpr int NC = M::NCP, NCT = NC / 16, MRT = 4;
-    __shared__ __align__(16) T xs[NC * kQLD];
-    __shared__ typename M::acc red[MRT * NCT][64];
-    const int lid = xcd_remap(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
-    const int e = lid / gridDim.x;
-    const int col0 = (lid % gridDim.x) * NC;
-    const int qpad = ent_info[6 * e], poff = ent_info[6 * e + 1];
-    const int np = ent_info[6 * e + 2], npad = ent_info[6 * e + 3];
-    const int nrt = npad / 16;
-    const T *ch = chir + ent_chi[e];
-    const int *gp = gpos + poff;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, lk = lane >> 4;
-    typename M::acc acc[MRT][NCT];
-#pragma unroll
-    for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) acc[rt][ct] = typename M::acc{0, 0, 0, 0};
-    for (int qc = 0; qc < qpad; qc += kQC) {
-        const int qn = min(kQC, qpad - qc);
-        // eight elements per thread at a time: point indices, then values,
-        // then stores (clamped: the tail repeats the last element)
-        for (int base = 0; base < qn * NC; base += 8 * 256) {
-            int cc[8], qq[8], gg[8];
-            T vv[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int t = min(base + (int)threadIdx.x + 256 * u, qn * NC - 1);
-                cc[u] = t / qn;
-                qq[u] = t - cc[u] * qn;
-                gg[u] = gp[qc + qq[u]];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const bool ok = gg[u] >= 0 && col0 + cc[u] < ncol;
-                vv[u] = X[ok ? (long)(col0 + cc[u]) * ldx + gg[u] : 0L];
-                if (!ok) vv[u] = T(0);
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) xs[cc[u] * kQLD + qq[u]] = vv[u];
-        }
-        __syncthreads();
-        const int qw = qn / 4;  // a multiple of 16
-        for (int k = wave * qw; k < (wave + 1) * qw; k += 16) {
-            // four k-steps: Chi loads first, then the MFMAs
-            T av[4][MRT];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const T *arow = ch + (long)(qc + k + 4 * u + lk) * npad + li;
-#pragma unroll
-                for (int rt = 0; rt < MRT; rt++) av[u][rt] = rt < nrt ? arow[rt * 16] : T(0);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int q = k + 4 * u + lk;
-                T bv[NCT];
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++) bv[ct] = xs[(ct * 16 + li) * kQLD + q];
-#pragma unroll
-                for (int rt = 0; rt < MRT; rt++) {
-                    if (rt < nrt) {
-#pragma unroll
-                        for (int ct = 0; ct < NCT; ct++) acc[rt][ct] = M::run(av[u][rt], bv[ct], acc[rt][ct]);
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // fixed-order cross-wave sum: wave 3 -> 2 -> 1 -> 0
-    for (int w = kWaves - 1; w >= 1; w--) {
-        if (wave == w)
-#pragma unroll
-            for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++) red[rt * NCT + ct][lane] = acc[rt][ct];
-        __syncthreads();
-        if (wave == w - 1)
-#pragma unroll
-            for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++) acc[rt][ct] += red[rt * NCT + ct][lane];
-        __syncthreads();
-    }
-    if (wave == 0) {
-#pragma unroll
-        for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-            for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int p = rt * 16 + M::drow(lk, r);
-                    const int col = col0 + ct * 16 + li;
-                    if (p < np && col < ncol) part[((long)e * max_np + p) * ncol + col] = acc[rt][ct][r];
-                }
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void nls_apply(T *__restrict__ out, long ldo, int ncol, int e0,
-                                                 const int *__restrict__ ent_info,
-                                                 const long *__restrict__ ent_chi,
-                                                 const int *__restrict__ gpos,
-                                                 const T *__restrict__ chit,
-                                                 const int *__restrict__ atom_img_ptr,
-                                                 const int *__restrict__ atom_img,
-                                                 const int *__restrict__ atom_row,
-                                                 const double *__restrict__ gamma,
-                                                 double scale_dv, const T *__restrict__ part,
-                                                 int max_np)
-{
-    using M = Mfma<T>;
-    constexpr int NC = M::NCA, NCT = NC / 16, LDB = NC * 3 / 2;
-    __shared__ T beta[64 * LDB];
-    const int lid = xcd_remap(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
-    const int e = e0 + lid / gridDim.x;
-    const int col0 = (lid % gridDim.x) * NC;
-    const int qpad = ent_info[6 * e], poff = ent_info[6 * e + 1];
-    const int np = ent_info[6 * e + 2], npad = ent_info[6 * e + 3], atom = ent_info[6 * e + 4];
-    const int i0 = atom_img_ptr[atom], i1 = atom_img_ptr[atom + 1], row = atom_row[atom];
-    // beta = scale dV Gamma sum over the atom's images of part, four
-    // elements per thread at a time with every load before the stores
-    // (clamped: the tail repeats the last element)
-    {
-        const int img0 = atom_img[i0];
-        for (int base = 0; base < npad * NC; base += 4 * 256) {
-            int pp[4], cc[4];
-            bool ok[4];
-            T vv[4];
-            double gm[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int t = min(base + (int)threadIdx.x + 256 * u, npad * NC - 1);
-                pp[u] = t / NC;
-                cc[u] = t - pp[u] * NC;
-                ok[u] = pp[u] < np && col0 + cc[u] < ncol;
-                vv[u] = part[ok[u] ? ((long)img0 * max_np + pp[u]) * ncol + col0 + cc[u] : 0L];
-                gm[u] = gamma[row + (ok[u] ? pp[u] : 0)];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                T v = ok[u] ? vv[u] : T(0);
-                if (ok[u]) {
-                    for (int i = i0 + 1; i < i1; i++)
-                        v += part[((long)atom_img[i] * max_np + pp[u]) * ncol + col0 + cc[u]];
-                    v *= (T)(scale_dv * gm[u]);
-                }
-                beta[pp[u] * LDB + cc[u]] = v;
-            }
-        }
-    }
-    __syncthreads();
-    const T *ct_ = chit + ent_chi[e];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, lk = lane >> 4;
-    for (int qt = wave; qt < qpad / 16; qt += kWaves) {
-        const int q0 = qt * 16;
-        // current output values loaded ahead of the MFMA chain
-        const int g = gpos[poff + q0 + li];
-        typename M::acc acc[NCT], ov[NCT];
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
-            acc[ct] = typename M::acc{0, 0, 0, 0};
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int col = col0 + ct * 16 + M::drow(lk, r);
-                ov[ct][r] = (g >= 0 && col < ncol) ? out[(long)col * ldo + g] : T(0);
-            }
-        }
-        for (int jb = 0; jb < npad; jb += 16) {
-            // npad is a multiple of 16: four p-steps, Chi loads first
-            T bqs[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) bqs[u] = ct_[(long)(jb + 4 * u + lk) * qpad + q0 + li];  // B (p, point)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = jb + 4 * u;
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++)                    // A (col, p)
-                    acc[ct] = M::run(beta[(j + lk) * LDB + ct * 16 + li], bqs[u], acc[ct]);
-            }
-        }
-        if (g < 0) continue;
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int col = col0 + ct * 16 + M::drow(lk, r);
-                if (col < ncol) out[(long)col * ldo + g] = ov[ct][r] + acc[ct][r];
-            }
-        }
-    }
-}
+//     sum_p Chi_e[q][p] beta[p][col].  Entries of one colour share no grid
+//     point, so the read-add-write needs no atomics and the result is
+//     deterministic.  In a Chebyshev chain (every Hamiltonian output is the
+//     next input) with one colour, an entry's points hold final values after
+//     its apply, and the same launch forms the next application's partials,
+//     into the other partials buffer (the atom's images still read this
+//     application's for beta); 1. then runs once per filter.
+//
+// A block is an entry and 16 columns; its eight waves take its 16-point tiles
+// in turn.  The apply is computed transposed (cols x points), so that a load or
+// store instruction covers 16 consecutive points of four columns; the result is
+// transposed through a wave-private LDS slice into the projection's B operand.
+// Every value that a group of GT tiles needs (the gathered block, Chi for both
+// products, beta) is loaded straight into its MFMA operand before the first
+// product, so a wave pays one memory latency per group.
+// What bounds it: with few entries that latency, with many the requests of the
+// 8- to 10-point runs (9.1 M of the 12.3 M writes of a 216-atom apply are
+// parts of 64 bytes).  Per application, fused: 26^3 x 24 FP32, 8 atoms: 8.5 us,
+// against 17.3 us for 256-thread blocks of 32 columns that staged beta and Chi
+// in LDS and had one tile's loads in flight; 78^3 x 480 FP32, 216 atoms: 456
+// against 495 us; 52^3 x 160 FP64, 64 atoms: 72 against 67 us (67 again in
+// column panels).  In three colours, 45 x 51 x 73 x 37 FP64: 10.5 against
+// 17.5 us a colour, the projection 8.5 against 22 us.
+constexpr int kEnt = 8;            // ints per entry in ent_info
+// Waves per block.  16 rather than 8, 12 or 4 where one projector tile leaves
+// the registers (at most 128): a whole entry is then one or two groups of
+// loads.  26^3 x 24 FP32, 8 atoms, per launch: 8.5 us, against 13.0 us with 8
+// waves.
+constexpr int nls_waves(int rt) { return rt == 1 ? 16 : 8; }
 
 // Orders a wavefront's LDS writes before its later LDS reads and the reads
 // before later writes, for data exchanged between lanes of one wave only:
@@ -1131,239 +948,160 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Chained applies (the Chebyshev recurrence, where every Hamiltonian output
-// is the next input), sphere layout with one colour (no two entries share a
-// grid point): after an entry's apply its points hold final values, so the
-// entry's partials for the next application are formed here from the tile
-// still in registers instead of re-gathering the block in nls_project.  Each
-// wave's 16-point x NC-column result is transposed through a wave-private
-// LDS slice into the MFMA B layout (points along k); Chi is the A operand
-// from the [p][qpad] copy.  The partials go to the other partials buffer
-// (the atom's images still read this application's partials for beta).
-// Wave w takes, chunk by chunk, the quarter of the points that nls_project
-// gives it, in the same order, and the waves are summed in the same fixed
-// order, so the partials are bitwise those of the unfused path.
-// The waves run independently between the beta staging and the final sum:
-// a tile's grid indices are read two tiles ahead and its current output
-// values one tile ahead, and all of a tile's Chi operands are issued before
-// its first MFMA.  MRT: 16-row projector tiles held (npad <= 16 MRT).  CHL:
-// each kQC-point chunk of the entry's Chi is first copied to LDS by the
-// whole block (coalesced 16-byte loads) and the operands are read there.
-template <typename T, int MRT, bool CHL>
-__global__ __launch_bounds__(256) void nls_apply_proj(T *__restrict__ out, long ldo, int ncol,
-                                                      int e0, const int *__restrict__ ent_info,
-                                                      const long *__restrict__ ent_chi,
-                                                      const int *__restrict__ gpos,
-                                                      const T *__restrict__ chit,
-                                                      const int *__restrict__ atom_img_ptr,
-                                                      const int *__restrict__ atom_img,
-                                                      const int *__restrict__ atom_row,
-                                                      const double *__restrict__ gamma,
-                                                      double scale_dv, const T *__restrict__ part,
-                                                      int max_np, T *__restrict__ part_next)
+// RT: 16-row projector tiles (npad <= 16 RT); APPLY / PROJ as above (out is
+// only read without APPLY).
+template <typename T, int RT, bool APPLY, bool PROJ>
+__global__ __launch_bounds__(64 * nls_waves(RT)) void nls_chain(
+    T *out, long ldo, int ncol, int e0, const int *__restrict__ ent_info,
+    const long *__restrict__ ent_chi, const int *__restrict__ gpos, const T *__restrict__ chir,
+    const T *__restrict__ chit, const int *__restrict__ atom_img, const double *__restrict__ gamma,
+    double scale_dv, const T *__restrict__ part, int max_np, T *__restrict__ part_next)
 {
     using M = Mfma<T>;
     using acc_t = typename M::acc;
-    constexpr int NC = M::NCA, NCT = NC / 16, LDB = NC * 3 / 2, LDY = NC + 1;
-    constexpr int LDQ = kQC + 16;  // LDS stride of a staged Chi row
-    __shared__ T beta[16 * MRT * LDB];
-    __shared__ T ytile[kWaves * 16 * LDY];
-    __shared__ acc_t red[MRT * NCT][64];
-    __shared__ __align__(16) T chs[CHL ? 16 * MRT * LDQ : 1];
+    constexpr int NW = nls_waves(RT), GT = sizeof(T) == 8 || RT > 2 ? 1 : RT == 2 ? 2 : 3, LDY = 17;
+    __shared__ T ytile[PROJ ? NW * 16 * LDY : 1];
+    __shared__ acc_t red[PROJ ? NW * RT : 1][64];
+    // the column blocks of one entry are consecutive logical ids -> one XCD
     const int lid = xcd_remap(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int e = e0 + lid / gridDim.x;
-    const int col0 = (lid % gridDim.x) * NC;
-    const int qpad = ent_info[6 * e], poff = ent_info[6 * e + 1];
-    const int np = ent_info[6 * e + 2], npad = ent_info[6 * e + 3], atom = ent_info[6 * e + 4];
-    const int nrt = npad / 16;
-    const int i0 = atom_img_ptr[atom], i1 = atom_img_ptr[atom + 1], row = atom_row[atom];
+    const int col0 = (lid % gridDim.x) * 16;
+    const int4 in0 = reinterpret_cast<const int4 *>(ent_info)[2 * e];
+    const int4 in1 = reinterpret_cast<const int4 *>(ent_info)[2 * e + 1];
+    const int qpad = in0.x, np = in0.z, npad = in0.w;
+    const int row = in1.x, img0 = in1.y, nimg = in1.z, iptr = in1.w;
+    const int *gp = gpos + in0.y;
+    const long choff = ent_chi[e];
+    const T *ct = chit + choff, *cr = chir + choff;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, lk = lane >> 4;
-    // the wave's tiles: chunk t / 4 of kQC points, tile t % 4 of the wave's
-    // quarter of the chunk (every chunk but the last holds four per wave)
-    const int ntile = qpad / 64;
-    auto tile_q0 = [&](int t) {
-        const int qc = (t >> 2) * kQC;
-        return qc + wave * (min(kQC, qpad - qc) >> 2) + (t & 3) * 16;
-    };
-    const int *gp = gpos + poff;
-    auto load_out = [&](acc_t *ov, int g) {
+    const int ntile = qpad / 16;
+    // beta: A (col, p), rows 4 s + lk of my column
+    T beta[APPLY ? 4 * RT : 1];
+    if constexpr (APPLY) {
+        const int col = col0 + li;
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int col = col0 + ct * 16 + M::drow(lk, r);
-                const bool ok = g >= 0 && col < ncol;
-                const T v = out[ok ? (long)col * ldo + g : 0L];
-                ov[ct][r] = ok ? v : T(0);
-            }
-    };
-    // the first tile's outputs are requested before the beta staging
-    int g_cur = gp[tile_q0(0) + li];
-    int g_nxt = ntile > 1 ? gp[tile_q0(1) + li] : -1;
-    acc_t ov[NCT];
-    load_out(ov, g_cur);
-    // beta = scale dV Gamma sum over the atom's images of part, four
-    // elements per thread at a time with every load before the stores
-    // (clamped: the tail repeats the last element)
-    {
-        const int img0 = atom_img[i0];
-        for (int base = 0; base < npad * NC; base += 4 * 256) {
-            int pp[4], cc[4];
-            bool ok[4];
-            T vv[4];
-            double gm[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int t = min(base + (int)threadIdx.x + 256 * u, npad * NC - 1);
-                pp[u] = t / NC;
-                cc[u] = t - pp[u] * NC;
-                ok[u] = pp[u] < np && col0 + cc[u] < ncol;
-                vv[u] = part[ok[u] ? ((long)img0 * max_np + pp[u]) * ncol + col0 + cc[u] : 0L];
-                gm[u] = gamma[row + (ok[u] ? pp[u] : 0)];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                T v = ok[u] ? vv[u] : T(0);
-                if (ok[u]) {
-                    for (int i = i0 + 1; i < i1; i++)
-                        v += part[((long)atom_img[i] * max_np + pp[u]) * ncol + col0 + cc[u]];
-                    v *= (T)(scale_dv * gm[u]);
-                }
-                beta[pp[u] * LDB + cc[u]] = v;
-            }
+        for (int s = 0; s < 4 * RT; s++) {
+            const int p = 4 * s + lk;
+            const bool ok = p < np && col < ncol;
+            T v = part[ok ? ((long)img0 * max_np + p) * ncol + col : 0L];
+            if (ok)
+                for (int i = 1; i < nimg; i++)
+                    v += part[((long)atom_img[iptr + i] * max_np + p) * ncol + col];
+            v *= (T)(scale_dv * gamma[row + (ok ? p : 0)]);
+            beta[s] = ok ? v : T(0);
         }
     }
-    __syncthreads();
-    const T *ct_ = chit + ent_chi[e];
+    // my result registers' columns
+    T *oc[4];
+    bool cok[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int col = col0 + M::drow(lk, r);
+        cok[r] = col < ncol;
+        oc[r] = out + (cok[r] ? (long)col * ldo : 0L);
+    }
+    acc_t pacc[PROJ ? RT : 1];
+#pragma unroll
+    for (int rt = 0; rt < (PROJ ? RT : 1); rt++) pacc[rt] = acc_t{0, 0, 0, 0};
     T *yw = ytile + wave * 16 * LDY;
-    acc_t pacc[MRT][NCT];
+    for (int tb = wave; tb < ntile; tb += NW * GT) {
+        int g[GT];
+        T ov[GT][4], bq[APPLY ? GT : 1][4 * RT], av[PROJ ? GT : 1][RT][4];
 #pragma unroll
-    for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) pacc[rt][ct] = acc_t{0, 0, 0, 0};
-    for (int t = 0; t < ntile; t++) {
-        const int q0 = tile_q0(t);
-        const int qc = (t >> 2) * kQC;
-        if (CHL && (t & 3) == 0) {
-            // stage Chi rows 0..npad of points qc .. qc + qn (all loads first)
-            using V = typename Vec16<T>::type;
-            constexpr int VW = sizeof(V) / sizeof(T), kS = 16 * MRT * kQC / VW / 256;
-            const int qv = min(kQC, qpad - qc) / VW, nv = npad * qv;
-            V v[kS];
-#pragma unroll
-            for (int j = 0; j < kS; j++) {
-                const int f = min((int)threadIdx.x + 256 * j, nv - 1);
-                const int pr = f / qv, qq = (f - pr * qv) * VW;
-                v[j] = *reinterpret_cast<const V *>(ct_ + (long)pr * qpad + qc + qq);
-            }
-            __syncthreads();  // the previous chunk's operands are read
-#pragma unroll
-            for (int j = 0; j < kS; j++) {
-                const int f = threadIdx.x + 256 * j;
-                if (f < nv) {
-                    const int pr = f / qv, qq = (f - pr * qv) * VW;
-                    *reinterpret_cast<V *>(chs + pr * LDQ + qq) = v[j];
-                }
-            }
-            __syncthreads();
+        for (int i = 0; i < GT; i++) {
+            // a group's tiles past the entry repeat its last one, without effect
+            const int t = tb + i * NW;
+            const int v = gp[min(t, ntile - 1) * 16 + li];
+            g[i] = t < ntile ? v : -1;
         }
-        // Chi operands of the tile: B (p, point) of the apply, A (p, point)
-        // of the projection (rows past npad are never read: nrt <= MRT)
-        T bq[MRT][4], av[4][MRT];
 #pragma unroll
-        for (int rt = 0; rt < MRT; rt++)
+        for (int i = 0; i < GT; i++) {
+            const int q0 = min(tb + i * NW, ntile - 1) * 16;
+            if constexpr (APPLY) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const bool ok = rt < nrt;
-                if (CHL) {
-                    const int ql = q0 - qc;
-                    bq[rt][u] = ok ? chs[(rt * 16 + 4 * u + lk) * LDQ + ql + li] : T(0);
-                    av[u][rt] = ok ? chs[(rt * 16 + li) * LDQ + ql + 4 * u + lk] : T(0);
-                } else {
-                    bq[rt][u] = ok ? ct_[(long)(rt * 16 + 4 * u + lk) * qpad + q0 + li] : T(0);
-                    av[u][rt] = ok ? ct_[(long)(rt * 16 + li) * qpad + q0 + 4 * u + lk] : T(0);
-                }
+                for (int s = 0; s < 4 * RT; s++)  // B (p, point); rows past npad: beta is zero
+                    bq[i][s] = ct[(long)min(4 * s + lk, npad - 1) * qpad + q0 + li];
             }
-        // the next tile's outputs, and the grid index of the one after
-        acc_t ovn[NCT];
-        load_out(ovn, t + 1 < ntile ? g_nxt : -1);
-        const int g_nn = t + 2 < ntile ? gp[tile_q0(t + 2) + li] : -1;
-        acc_t acc[NCT];
+            if constexpr (PROJ) {
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) acc[ct] = acc_t{0, 0, 0, 0};
+                for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-        for (int rt = 0; rt < MRT; rt++) {
-            if (rt < nrt) {
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int j = rt * 16 + 4 * u;
-#pragma unroll
-                    for (int ct = 0; ct < NCT; ct++)
-                        acc[ct] = M::run(beta[(j + lk) * LDB + ct * 16 + li], bq[rt][u], acc[ct]);
-                }
+                    for (int u = 0; u < 4; u++)  // A (p, point); rows past np are not stored
+                        av[i][rt][u] = cr[(long)(q0 + 4 * u + lk) * npad + min(rt * 16 + li, npad - 1)];
             }
         }
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
+        for (int i = 0; i < GT; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int cl = ct * 16 + M::drow(lk, r);
-                const bool ok = g_cur >= 0 && col0 + cl < ncol;
-                const T y = ov[ct][r] + acc[ct][r];
-                if (ok) out[(long)(col0 + cl) * ldo + g_cur] = y;
-                yw[li * LDY + cl] = ok ? y : T(0);
+                const T v = oc[r][max(g[i], 0)];
+                ov[i][r] = g[i] >= 0 && cok[r] ? v : T(0);
             }
-        }
-        wave_lds_order();
 #pragma unroll
-        for (int s4 = 0; s4 < 4; s4++) {
-            T bv[NCT];
+        for (int i = 0; i < GT; i++) {
+            if constexpr (APPLY) {
+                acc_t acc = acc_t{0, 0, 0, 0};
 #pragma unroll
-            for (int ct = 0; ct < NCT; ct++) bv[ct] = yw[(4 * s4 + lk) * LDY + ct * 16 + li];
-#pragma unroll
-            for (int rt = 0; rt < MRT; rt++) {
-                if (rt < nrt) {
-#pragma unroll
-                    for (int ct = 0; ct < NCT; ct++)
-                        pacc[rt][ct] = M::run(av[s4][rt], bv[ct], pacc[rt][ct]);
-                }
-            }
-        }
-        wave_lds_order();
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) ov[ct] = ovn[ct];
-        g_cur = g_nxt;
-        g_nxt = g_nn;
-    }
-    // fixed-order cross-wave sum: wave 3 -> 2 -> 1 -> 0
-    for (int w = kWaves - 1; w >= 1; w--) {
-        if (wave == w)
-#pragma unroll
-            for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++) red[rt * NCT + ct][lane] = pacc[rt][ct];
-        __syncthreads();
-        if (wave == w - 1)
-#pragma unroll
-            for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-                for (int ct = 0; ct < NCT; ct++) pacc[rt][ct] += red[rt * NCT + ct][lane];
-        __syncthreads();
-    }
-    if (wave == 0) {
-#pragma unroll
-        for (int rt = 0; rt < MRT; rt++)
-#pragma unroll
-            for (int ct = 0; ct < NCT; ct++)
+                for (int s = 0; s < 4 * RT; s++) acc = M::run(beta[s], bq[i][s], acc);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const int p = rt * 16 + M::drow(lk, r);
-                    const int col = col0 + ct * 16 + li;
-                    if (p < np && col < ncol)
-                        part_next[((long)e * max_np + p) * ncol + col] = pacc[rt][ct][r];
+                    const T y = ov[i][r] + acc[r];
+                    const bool ok = g[i] >= 0 && cok[r];
+                    if (ok) oc[r][g[i]] = y;
+                    ov[i][r] = ok ? y : T(0);
                 }
+            }
+            if constexpr (PROJ) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) yw[li * LDY + M::drow(lk, r)] = ov[i][r];
+                wave_lds_order();
+                T bv[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) bv[u] = yw[(4 * u + lk) * LDY + li];
+                wave_lds_order();
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) pacc[rt] = M::run(av[i][rt][u], bv[u], pacc[rt]);
+            }
+        }
     }
+    if constexpr (PROJ) {
+        // the waves' sums in wave order
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) red[wave * RT + rt][lane] = pacc[rt];
+        __syncthreads();
+        if (wave < RT) {
+            acc_t sum = red[wave][lane];
+            for (int w = 1; w < NW; w++) sum += red[w * RT + wave][lane];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int p = wave * 16 + M::drow(lk, r);
+                const int col = col0 + li;
+                if (p < np && col < ncol) part_next[((long)e * max_np + p) * ncol + col] = sum[r];
+            }
+        }
+    }
+}
+
+// One nls_chain launch over ne entries from e0.
+template <typename T, bool APPLY, bool PROJ>
+int launch_nls(sgpu_context *ctx, int ncol, T *out, long ldo, int e0, int ne, const T *chir, const T *chit,
+               double scale_dv, const T *part, T *part_next)
+{
+    const sgpu_nonlocal &nl = ctx->nl;
+    const dim3 grid((ncol + 15) / 16, ne);
+    auto go = [&](auto kern, int waves) {
+        kern<<<grid, 64 * waves, 0, ctx->stream>>>(out, ldo, ncol, e0, nl.ent_info, nl.ent_chi, nl.gpos,
+                                                       chir, chit, nl.atom_img, nl.gamma, scale_dv, part,
+                                                       64, part_next);
+    };
+    if (nl.max_npad <= 16) go(nls_chain<T, 1, APPLY, PROJ>, nls_waves(1));
+    else if (nl.max_npad <= 32) go(nls_chain<T, 2, APPLY, PROJ>, nls_waves(2));
+    else go(nls_chain<T, 4, APPLY, PROJ>, nls_waves(4));
+    SGPU_HIP(hipGetLastError());
+    return SGPU_OK;
 }
 
 // SPARC_AMD_NLB=lds selects the LDS-staged nlb_project and the transposed
@@ -1505,25 +1243,20 @@ int launch_vnl_sphere(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out,
                       double scale, const T *chir, const T *chit, void *ws, size_t ws_bytes)
 {
     const sgpu_nonlocal &nl = ctx->nl;
-    constexpr int NCP = Mfma<T>::NCP, NC = Mfma<T>::NCA;
-    const int max_np = 64;
     void *buf = nullptr;
     SGPU_CHECK(vnl_partials(ctx, sizeof(T) == 4 ? SGPU_F32 : SGPU_F64, ncol, ws, ws_bytes, &buf));
     T *part = (T *)buf;
     sgpu_tmark t;
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    nls_project<T><<<dim3((ncol + NCP - 1) / NCP, nl.n_ent), 256, 0, ctx->stream>>>(
-        x, ldx, ncol, nl.ent_info, nl.ent_chi, nl.gpos, chir, max_np, part);
-    SGPU_HIP(hipGetLastError());
+    SGPU_CHECK((launch_nls<T, false, true>(ctx, ncol, const_cast<T *>(x), ldx, 0, nl.n_ent, chir, chit, 0.0,
+                                           nullptr, part)));
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
     for (int c = 0; c < nl.n_colors; c++) {
         const int e0 = nl.color_start[c], ne = nl.color_start[c + 1] - e0;
         if (ne <= 0) continue;
-        nls_apply<T><<<dim3((ncol + NC - 1) / NC, ne), 256, 0, ctx->stream>>>(
-            out, ldo, ncol, e0, nl.ent_info, nl.ent_chi, nl.gpos, chit, nl.atom_img_ptr,
-            nl.atom_img, nl.atom_row, nl.gamma, scale * nl.dV, part, max_np);
-        SGPU_HIP(hipGetLastError());
+        SGPU_CHECK((launch_nls<T, true, false>(ctx, ncol, out, ldo, e0, ne, chir, chit, scale * nl.dV, part,
+                                               nullptr)));
     }
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
     return SGPU_OK;
@@ -1583,9 +1316,7 @@ int launch_vnl_chain_sphere(sgpu_context *ctx, int ncol, const T *x, long ldx, T
     sgpu_nonlocal &nl = ctx->nl;
     *projected = false;
     if (nl.n_ent == 0 || ncol <= 0) return SGPU_OK;
-    constexpr int NCP = Mfma<T>::NCP, NC = Mfma<T>::NCA;
-    const int max_np = 64;
-    const size_t part_elems = (size_t)nl.n_ent * max_np * ncol;
+    const size_t part_elems = (size_t)nl.n_ent * 64 * ncol;
     const size_t need = 2 * part_elems * sizeof(T) + 256;
     if (have_part && need > nl.chain_bytes) {
         sgpu_set_error("nonlocal chain: partials of a different shape");
@@ -1599,38 +1330,22 @@ int launch_vnl_chain_sphere(sgpu_context *ctx, int ncol, const T *x, long ldx, T
     sgpu_tmark t;
     if (!have_part) {
         SGPU_CHECK(sgpu_tbegin(ctx, &t));
-        nls_project<T><<<dim3((ncol + NCP - 1) / NCP, nl.n_ent), 256, 0, ctx->stream>>>(
-            x, ldx, ncol, nl.ent_info, nl.ent_chi, nl.gpos, chir, max_np, part);
-        SGPU_HIP(hipGetLastError());
+        SGPU_CHECK((launch_nls<T, false, true>(ctx, ncol, const_cast<T *>(x), ldx, 0, nl.n_ent, chir, chit,
+                                               0.0, nullptr, part)));
         SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     }
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
     if (want_next && nl.n_colors == 1) {
-        const dim3 grid((ncol + NC - 1) / NC, nl.n_ent);
-        auto go = [&](auto kern) {
-            kern<<<grid, 256, 0, ctx->stream>>>(out, ldo, ncol, 0, nl.ent_info, nl.ent_chi,
-                                                nl.gpos, chit, nl.atom_img_ptr, nl.atom_img,
-                                                nl.atom_row, nl.gamma, scale * nl.dV, part,
-                                                max_np, part_next);
-        };
-        // Chi staged in LDS for FP32 with up to 32 projector rows (53 KB of
-        // LDS per block, three blocks per CU); FP64 reads it from L2
-        constexpr bool F32 = sizeof(T) == 4;
-        if (nl.max_npad <= 32)
-            go(nls_apply_proj<T, 2, F32>);
-        else
-            go(nls_apply_proj<T, 4, false>);
-        SGPU_HIP(hipGetLastError());
+        SGPU_CHECK((launch_nls<T, true, true>(ctx, ncol, out, ldo, 0, nl.n_ent, chir, chit, scale * nl.dV,
+                                              part, part_next)));
         nl.chain_cur ^= 1;
         *projected = true;
     } else {
         for (int c = 0; c < nl.n_colors; c++) {
             const int e0 = nl.color_start[c], ne = nl.color_start[c + 1] - e0;
             if (ne <= 0) continue;
-            nls_apply<T><<<dim3((ncol + NC - 1) / NC, ne), 256, 0, ctx->stream>>>(
-                out, ldo, ncol, e0, nl.ent_info, nl.ent_chi, nl.gpos, chit, nl.atom_img_ptr,
-                nl.atom_img, nl.atom_row, nl.gamma, scale * nl.dV, part, max_np);
-            SGPU_HIP(hipGetLastError());
+            SGPU_CHECK((launch_nls<T, true, false>(ctx, ncol, out, ldo, e0, ne, chir, chit, scale * nl.dV,
+                                                   part, nullptr)));
         }
     }
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
@@ -1704,7 +1419,7 @@ int upload(T **dst, const T *src, size_t n, hipStream_t s)
     return SGPU_OK;
 }
 
-// Sphere layout (see nls_project / nls_apply): entries greedily coloured so
+// Sphere layout (see nls_chain): entries greedily coloured so
 // that no two entries of a colour share a grid point, each entry's point
 // list padded to a multiple of 64 (-1 = padding) and its Chi stored twice,
 // [q][npad] for the projection and [p][qpad] for the apply.
@@ -1740,12 +1455,25 @@ int build_sphere_layout(sgpu_context *ctx, int n_influence, const int *ndc, cons
     }
     std::vector<int> order(n_influence);
     std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return color[x] < color[y]; });
+    // within a colour along x, then y, then z (in steps of a sphere's size, by
+    // the middle point): a 128-byte line holds points of neighbouring spheres,
+    // and blocks that run together then find it in their XCD's L2
+    constexpr int bin = 8;
+    std::vector<long> place(n_influence, 0);
+    for (int a = 0; a < n_influence; a++)
+        if (ndc[a] > 0) {
+            const int q = grid_pos[pos_off[a] + ndc[a] / 2];
+            const int ix = q % ctx->nx, iy = (q / ctx->nx) % ctx->ny, iz = q / (ctx->nx * ctx->ny);
+            place[a] = ((long)(iz / bin) * ctx->ny + iy / bin) * ctx->nx + ix;
+        }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return color[x] != color[y] ? color[x] < color[y] : place[x] < place[y];
+    });
     std::vector<int> color_start(n_colors + 1, 0);
     for (int a = 0; a < n_influence; a++) color_start[color[a] + 1]++;
     for (int c = 0; c < n_colors; c++) color_start[c + 1] += color_start[c];
     // per entry layout
-    std::vector<int> info(6 * (size_t)n_influence), gp;
+    std::vector<int> info(kEnt * (size_t)n_influence), gp;
     std::vector<long> eoff(n_influence);
     std::vector<double> chir, chit;
     std::vector<std::vector<int>> imgs(n_atoms);
@@ -1756,12 +1484,11 @@ int build_sphere_layout(sgpu_context *ctx, int n_influence, const int *ndc, cons
         const int n = ndc[a], np = nproj[a];
         const int qpad = std::max(64, (n + 63) / 64 * 64), npad = std::max(16, (np + 15) / 16 * 16);
         const int atom = atom_of(a);
-        info[6 * e] = qpad;
-        info[6 * e + 1] = (int)gp.size();
-        info[6 * e + 2] = np;
-        info[6 * e + 3] = npad;
-        info[6 * e + 4] = atom;
-        info[6 * e + 5] = 0;
+        info[kEnt * e] = qpad;
+        info[kEnt * e + 1] = (int)gp.size();
+        info[kEnt * e + 2] = np;
+        info[kEnt * e + 3] = npad;
+        info[kEnt * e + 4] = alpha_off[a];
         eoff[e] = coff;
         imgs[atom].push_back(e);
         max_qpad = std::max(max_qpad, qpad);
@@ -1777,11 +1504,22 @@ int build_sphere_layout(sgpu_context *ctx, int n_influence, const int *ndc, cons
             }
         coff += (long)qpad * npad;
     }
+    // an atom's images in the order they were given, whatever the entries' order
+    for (auto &v : imgs)
+        std::sort(v.begin(), v.end(), [&](int x, int y) {
+            return color[order[x]] != color[order[y]] ? color[order[x]] < color[order[y]]
+                                                      : order[x] < order[y];
+        });
     std::vector<int> img_ptr(n_atoms + 1, 0), img, arow(n_atoms);
     for (int t = 0; t < n_atoms; t++) {
         img_ptr[t + 1] = img_ptr[t] + (int)imgs[t].size();
         img.insert(img.end(), imgs[t].begin(), imgs[t].end());
         arow[t] = offs[t];
+        for (int e : imgs[t]) {  // the atom's images: first, number, place in img
+            info[kEnt * e + 5] = imgs[t][0];
+            info[kEnt * e + 6] = (int)imgs[t].size();
+            info[kEnt * e + 7] = img_ptr[t];
+        }
     }
     sgpu_nonlocal &nl = ctx->nl;
     hipStream_t s = ctx->stream;
@@ -1879,7 +1617,7 @@ __global__ void nls_sum_images(const T *__restrict__ part, int ncol, int n_atoms
     const long ap = t / ncol;
     const int p = (int)(ap % max_np), a = (int)(ap / max_np);
     const int i0 = atom_img_ptr[a], i1 = atom_img_ptr[a + 1];
-    if (p >= ent_info[6 * atom_img[i0] + 2]) return;
+    if (p >= ent_info[kEnt * atom_img[i0] + 2]) return;
     double v = 0.0;
     for (int i = i0; i < i1; i++) v += (double)part[((long)atom_img[i] * max_np + p) * ncol + col];
     alpha[(long)(atom_row[a] + p) * ncol + col] = (T)(scale * v);
@@ -1896,10 +1634,10 @@ int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scal
         const int max_np = 64;
         SGPU_CHECK(sgpu_scratch(ctx, (size_t)nl.n_ent * max_np * ncol * sizeof(T) + 256, &buf));
         T *part = (T *)buf;
-        nls_project<T><<<dim3((ncol + NCP - 1) / NCP, nl.n_ent), 256, 0, ctx->stream>>>(
-            x, ldx, ncol, nl.ent_info, nl.ent_chi, nl.gpos,
-            sizeof(T) == 8 ? (const T *)nl.chir64 : (const T *)nl.chir32, max_np, part);
-        SGPU_HIP(hipGetLastError());
+        const T *chir = sizeof(T) == 8 ? (const T *)nl.chir64 : (const T *)nl.chir32;
+        const T *chit = sizeof(T) == 8 ? (const T *)nl.chit64 : (const T *)nl.chit32;
+        SGPU_CHECK((launch_nls<T, false, true>(ctx, ncol, const_cast<T *>(x), ldx, 0, nl.n_ent, chir, chit,
+                                               0.0, nullptr, part)));
         const long total = (long)nl.n_atoms * max_np * ncol;
         nls_sum_images<T><<<(unsigned)((total + 255) / 256), 256, 0, ctx->stream>>>(
             part, ncol, nl.n_atoms, max_np, nl.atom_img_ptr, nl.atom_img, nl.atom_row, nl.ent_info,

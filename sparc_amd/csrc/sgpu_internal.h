@@ -85,7 +85,8 @@ struct sgpu_nonlocal {
     long stored = 0;            // projector values per copy, zero padding included
     int n_ent = 0, n_atoms = 0, n_colors = 0, max_qpad = 0, max_npad = 0;
     std::vector<int> color_start;   // host: first entry of each colour (+ end)
-    int *ent_info = nullptr;    // per entry: qpad, pos offset, np, npad, atom, chi offset (6 ints)
+    int *ent_info = nullptr;    // per entry: qpad, pos offset, np, npad, alpha row, first image,
+                                // number of images, their place in atom_img (8 ints)
     long *ent_chi = nullptr;    // per entry: element offset of its Chi blocks
     int *gpos = nullptr;        // grid index per padded point (-1: padding)
     double *chir64 = nullptr;   // Chi [q][npad] per entry

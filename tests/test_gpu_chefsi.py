@@ -327,6 +327,47 @@ def test_brick_chain_edges(gpu, oracle_mod, monkeypatch, n, sites, lmax, ncol, d
     assert rel_err(out["1"], Yo) < (1e-11 if dtype == 0 else 1e-4)
 
 
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("rc,lmax,nsig,ncol", [
+    (0.6, 0, 1, 1),     # a handful of points, one row, one column
+    (2.4, 1, 2, 17),    # 8 rows, more point tiles than waves
+    (1.9, 2, 2, 33),    # 18 rows: two row tiles
+    (2.4, 2, 4, 16),    # 36 rows: four row tiles, the last empty
+])
+def test_sphere_chain_edges(gpu, oracle_mod, monkeypatch, rc, lmax, nsig, ncol, dtype):
+    """The sphere layout's projection, apply and their fused form over row
+    tiles, point groups and column remainders, entries listed out of place
+    order and one atom split into images: the Chebyshev filter (fused) equal
+    to the unfused one, and both against the oracle.  Tolerances as in
+    test_filter_nonlocal_chain."""
+    from sparc_amd.workloads import Grid, gaussian_projectors, gaussian_veff
+    from tests.helpers import split_images
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "sphere")
+    g = Grid(21, 20, 18, 0.5, 0.5, 0.5)
+    rng = np.random.default_rng(71)
+    veff = gaussian_veff(g, 4, rng)
+    sites = np.array([[2.5, 7.5, 6.5], [7.6, 2.5, 2.5], [0.2, 2.5, 7.0]])
+    nl = split_images(gaussian_projectors(g, sites, rc, sigmas=(1.0, 0.7, 0.5, 1.3)[:nsig],
+                                          gammas=(1.3, -0.6, 0.4, -0.2)[:nsig], lmax=lmax), 2)
+    o = oracle_mod.Oracle(g, veff, nl)
+    a0, b, a = _bounds(o, g)
+    X = rng.uniform(-0.5, 0.5, (g.nd, ncol))
+    Yo, _ = o.chebyshev_filter(X, 4, a, b, a0)
+    out = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("SPARC_AMD_NL_CHAIN", chain)
+        with gpu.Context(g) as ctx:
+            ctx.set_veff(veff)
+            ctx.set_nonlocal(nl)
+            assert ctx.nonlocal_layout()[0] == 1
+            bx = ctx.block(ncol, dtype).upload(X)
+            by = ctx.block(ncol, dtype)
+            ctx.chebyshev_filter_dev(bx, by, 4, a, b, a0)
+            out[chain] = by.download()
+    assert np.array_equal(out["1"], out["0"])
+    assert rel_err(out["1"], Yo) < (1e-11 if dtype == 0 else 1e-4)
+
+
 @pytest.mark.parametrize("n,groups,threads", [(181, 32, 256), (300, 7, 256), (480, 32, 256),
                                               (480, 64, 512), (1000, 16, 256)])
 def test_generalized_eigensolve_cooperative_tridiagonal(gpu, monkeypatch, n, groups, threads):
