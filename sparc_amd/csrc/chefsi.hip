@@ -86,34 +86,61 @@ int apply_h_chain(sgpu_context *ctx, int dtype, int ncol, double c, const void *
     return SGPU_OK;
 }
 
+// Columns that a filter takes at a time: with the sphere layout in one colour,
+// panels whose two buffers stay in the 256 MB Infinity Cache over all degrees
+// (at most 96 MB each, equal, in multiples of 8), where the block itself is too
+// large for that.  Degree 20: 78^3 x 480 FP32, 216 atoms, 23.4 -> 19.3 ms (10
+// panels of 48; of 64, 121 MB, 20.7, of 32 22.5), 64 atoms 17.3 -> 14.7; 96^3 x
+// 256 FP32, 216 atoms, 19.0 -> 15.3; 52^3 x 160 FP64, 64 atoms, 3.82 -> 3.40;
+// 78^3 x 72 FP32 (137 MB) 3.41 -> 3.25, but x 64 (121 MB) in halves 2.81 ->
+// 2.87.  With fewer than 128 blocks in the nonlocal launches (52^3 x 170 FP64,
+// 8 atoms: 2.94 -> 3.15) or in several colours (40^3 x 512 FP64, 27 atoms: 6.5
+// -> 7.3) the shorter launches cost more than the cache gives; so do they in
+// the brick layout, whose blocks take 128 columns (96^3 x 512: 59 -> 62).
+int filter_panel(sgpu_context *ctx, int dtype, int ncol)
+{
+    const sgpu_nonlocal &nl = ctx->nl;
+    const double bytes = (double)ctx->nd * ncol * (dtype == SGPU_F64 ? 8 : 4);
+    if (nl.mode != 1 || nl.n_colors != 1 || !ctx->nl_chain || bytes < 136e6) return ncol;
+    const int np = (int)(bytes / 96e6) + 1;
+    const int panel = ((ncol + np - 1) / np + 7) / 8 * 8;
+    return (long)nl.n_ent * ((panel + 15) / 16) < 128 ? ncol : std::min(panel, ncol);
+}
+
 // Chebyshev filter on raw device storage (ChebyshevFiltering,
-// src/eigenSolver.c:722-798).  On return *res points at the buffer holding
-// Y_m and *prev at the one holding Y_{m-1}; bx starts as X, by as Y.
+// src/eigenSolver.c:722-798), a panel of columns at a time.  On return *res
+// points at the buffer holding Y_m and *prev at the one holding Y_{m-1}; bx
+// starts as X, by as Y.
 int filter_raw(sgpu_context *ctx, int dtype, int ncol, void *bx, void *by, long ld, int m,
                double a, double b, double a0, void **res, void **prev)
 {
     const double e = 0.5 * (b - a), c = 0.5 * (b + a);
-    double sigma = e / (a0 - c);
-    const double sigma1 = sigma, gamma = 2.0 / sigma1;
+    const double sigma1 = e / (a0 - c), gamma = 2.0 / sigma1;
+    const size_t colbytes = (size_t)ld * (dtype == SGPU_F64 ? 8 : 4);
+    const int panel = filter_panel(ctx, dtype, ncol);
     sgpu_tmark tall;
     SGPU_CHECK(sgpu_tbegin(ctx, &tall));
-    // Y = (sigma1 / e) (H - c) X
-    bool have_part = false;
-    SGPU_CHECK(apply_h_chain(ctx, dtype, ncol, -c, bx, ld, by, ld, nullptr, 0, sigma1 / e, 0.0,
-                             &have_part, m > 1));
-    void *P = by, *Q = bx;
-    for (int j = 1; j < m; j++) {
-        const double sigma2 = 1.0 / (gamma - sigma);
-        const double vs = 2.0 * sigma2 / e, vs2 = sigma * sigma2;
-        // Q <- vs (H - c) P - vs2 Q   (in place over Y_{j-1})
-        SGPU_CHECK(apply_h_chain(ctx, dtype, ncol, -c, P, ld, Q, ld, Q, ld, vs, -vs2, &have_part,
-                                 j + 1 < m));
-        std::swap(P, Q);
-        sigma = sigma2;
+    for (int c0 = 0; c0 < ncol; c0 += panel) {
+        const int nc = std::min(panel, ncol - c0);
+        void *P = (char *)by + c0 * colbytes, *Q = (char *)bx + c0 * colbytes;
+        double sigma = sigma1;
+        // Y = (sigma1 / e) (H - c) X
+        bool have_part = false;
+        SGPU_CHECK(apply_h_chain(ctx, dtype, nc, -c, Q, ld, P, ld, nullptr, 0, sigma1 / e, 0.0,
+                                 &have_part, m > 1));
+        for (int j = 1; j < m; j++) {
+            const double sigma2 = 1.0 / (gamma - sigma);
+            const double vs = 2.0 * sigma2 / e, vs2 = sigma * sigma2;
+            // Q <- vs (H - c) P - vs2 Q   (in place over Y_{j-1})
+            SGPU_CHECK(apply_h_chain(ctx, dtype, nc, -c, P, ld, Q, ld, Q, ld, vs, -vs2, &have_part,
+                                     j + 1 < m));
+            std::swap(P, Q);
+            sigma = sigma2;
+        }
     }
     SGPU_CHECK(sgpu_tend(ctx, &tall, "filter"));
-    *res = P;
-    *prev = Q;
+    *res = m % 2 ? by : bx;
+    *prev = m % 2 ? bx : by;
     return SGPU_OK;
 }
 

@@ -368,6 +368,39 @@ def test_sphere_chain_edges(gpu, oracle_mod, monkeypatch, rc, lmax, nsig, ncol, 
     assert rel_err(out["1"], Yo) < (1e-11 if dtype == 0 else 1e-4)
 
 
+@pytest.mark.parametrize("dtype,ncol,m", [(0, 135, 3), (1, 250, 4)])
+def test_filter_column_panels(gpu, oracle_mod, monkeypatch, dtype, ncol, m):
+    """A block too large for the Infinity Cache is filtered in panels of
+    columns (here 72 + 63 and 128 + 122): columns on both sides of the seam and
+    the last ones equal those of a narrow block, for odd and even degrees (the
+    result is in either buffer), and both buffers hold what the recurrence
+    leaves.  No operation crosses columns, so only the order of sums can
+    differ: 1e-13 / 1e-5 over 4 applications."""
+    from sparc_amd.workloads import Grid, gaussian_projectors, gaussian_veff
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "sphere")
+    g = Grid(52, 52, 52, 0.5, 0.5, 0.5)
+    rng = np.random.default_rng(77)
+    veff = gaussian_veff(g, 4, rng)
+    c = np.arange(4) * 6.5 + 3.0
+    sites = np.stack(np.meshgrid(c, c, c, indexing="ij"), -1).reshape(-1, 3)
+    nl = gaussian_projectors(g, sites, 1.6, sigmas=(1.0,), gammas=(1.3,), lmax=1)
+    a0, a, b = -1.0, 2.0, 60.0
+    X = rng.uniform(-0.5, 0.5, (g.nd, ncol))
+    cols = np.r_[0, 60:75, 120:ncol:1][-40:]
+    res = []
+    with gpu.Context(g) as ctx:
+        ctx.set_veff(veff)
+        ctx.set_nonlocal(nl)
+        for Z in (X, X[:, cols]):
+            bx = ctx.block(Z.shape[1], dtype).upload(Z)
+            by = ctx.block(Z.shape[1], dtype)
+            ctx.chebyshev_filter_dev(bx, by, m, a, b, a0)
+            res.append((by.download(), bx.download()))
+            bx.free(); by.free()
+    for whole, part in zip(*res):
+        assert rel_err(whole[:, cols], part) < (1e-13 if dtype == 0 else 1e-5)
+
+
 @pytest.mark.parametrize("n,groups,threads", [(181, 32, 256), (300, 7, 256), (480, 32, 256),
                                               (480, 64, 512), (1000, 16, 256)])
 def test_generalized_eigensolve_cooperative_tridiagonal(gpu, monkeypatch, n, groups, threads):
