@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "sgpu_internal.h"
+#include "wave_sum.h"
 
 namespace {
 
@@ -1085,135 +1086,152 @@ __device__ __forceinline__ void wave_sum_f64(double (&d)[CW])
 }
 
 // Householder reduction of a symmetric matrix to tridiagonal form inside one
-// workgroup, the matrix held in LDS: LAPACK dsytd2 with UPLO = 'L' (the
-// storage rocsolver_dormtr reads back): for i = 0..n-2, H(i) = I - tau v v'
-// with v(0:i) = 0, v(i+1) = 1 and v(i+2:n) stored in A(i+2:n, i); e(i) =
-// beta, d(i) = A(i,i).  Each step is dlarfg (beta = -sign(alpha) |(alpha, x)|,
-// tau = (beta - alpha) / beta, x /= alpha - beta), w = tau A22 v,
-// w -= (tau / 2)(w'v) v and the rank-2 update A22 -= v w' + w v' on the lower
-// triangle.  rocsolver's dsytrd takes ~1,800 dependent kernels for n = 480
-// (3.7 us each on the device); here every step is a few workgroup barriers.
-// The lower triangle is packed by columns: A(r, c), r >= c, at
-// c (2n - c + 1) / 2 + (r - c).  Sums use a fixed order (deterministic).
-constexpr int kTridMaxN = 180;   // packed triangle + work vectors fit in 160 KB of LDS
-constexpr int kTridThreads = 1024;
+// workgroup: LAPACK dsytd2 with UPLO = 'L' (the storage rocsolver_dormtr reads
+// back): for i = 0..n-2, H(i) = I - tau v v' with v(0:i) = 0, v(i+1) = 1 and
+// v(i+2:n) stored in A(i+2:n, i); e(i) = beta, d(i) = A(i,i).  Each step is
+// dlarfg (beta = -sign(alpha) |(alpha, x)|, tau = (beta - alpha) / beta, x /=
+// alpha - beta), w = tau A22 v - (tau^2 / 2) (v'A22 v) v and the rank-2 update
+// A22 -= v w' + w v'.
+// What bounds it: the chain of n dependent steps on one CU.  The matrix (both
+// triangles) stays in registers, row r in wave r mod 8, column c in lane c mod
+// 64, so the products with v and w need no LDS reads: v and w live in the same
+// lanes as the columns (every wave forms them itself, with the same bits) and
+// a row's two factors are read from their lanes.  A step then has one barrier:
+// the update also forms p = A22 v of the next step (its v follows from row
+// i + 1 alone), and p and the next row go to all waves through LDS.  n = 160:
+// 370 us, against 951 us for 1,024 threads with the packed triangle in LDS and
+// seven barriers a step.  Eight waves: with sixteen the vectors formed by
+// every wave would take twice the issue slots, with four the rows would not
+// fit in the registers.
+constexpr int kTridMaxN = 180;   // three columns a lane (144 registers of matrix)
+constexpr int kTridWaves = 8;
 
-__device__ __forceinline__ int tri_at(int n, int r, int c) { return c * (2 * n - c + 1) / 2 + (r - c); }
-
-// Sum over the workgroup in a fixed order (DPP wave sums, then the 16 wave
-// sums in order); the total is valid in thread 0.
-__device__ __forceinline__ double tri_block_sum(double v, double *red)
+template <int NQ>
+__global__ __launch_bounds__(64 * kTridWaves) void sytd2_lower_regs(double *__restrict__ A, int lda,
+                                                                    int n, double *__restrict__ D,
+                                                                    double *__restrict__ E,
+                                                                    double *__restrict__ tau)
 {
-    double a[1] = {v};
-    wave_sum_f64<1>(a);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a[0];
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int k = 0; k < kTridThreads / 64; k++) s += red[k];
-    return s;
-}
-
-__global__ __launch_bounds__(kTridThreads) void sytd2_lower_lds(double *__restrict__ A, int lda,
-                                                                  int n, double *__restrict__ D,
-                                                                  double *__restrict__ E,
-                                                                  double *__restrict__ tau)
-{
-    extern __shared__ double sm[];
-    const int npk = n * (n + 1) / 2;
-    double *P = sm;                 // packed lower triangle
-    double *v = P + npk;            // Householder vector of the current step (n)
-    double *w = v + n;              // w (n)
-    double *part = w + n;           // partial sums (kTridThreads)
-    __shared__ double sc[4];        // tau, scale, beta, dot
-    const int t = threadIdx.x;
-    for (int e = t; e < n * n; e += kTridThreads) {
-        const int c = e / n, r = e - c * n;
-        if (r >= c) P[tri_at(n, r, c)] = A[(long)c * lda + r];
+    constexpr int NK = 64 * NQ / kTridWaves;   // rows per wave
+    __shared__ double ps[2][64 * NQ], rs[2][64 * NQ];  // p and row i + 1, by step parity
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+    double a[NK][NQ], v[NQ], w[NQ], x[NQ];
+#pragma unroll
+    for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int r = wv + kTridWaves * k, c = ln + 64 * q;
+            const int hi = max(r, c), lo = min(r, c);
+            const double e = A[min(lo, n - 1) * lda + min(hi, n - 1)];
+            a[k][q] = hi < n ? e : 0.0;
+            if (q == NQ - 1 && k % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few addresses at a time
+        }
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        const int c = ln + 64 * q;
+        x[q] = c >= 1 && c < n ? A[c] : 0.0;
+        v[q] = w[q] = 0.0;
     }
-    __syncthreads();
-    for (int i = 0; i + 1 < n; i++) {
-        const int m = n - i - 1;               // length of x = A(i+1:n, i)
-        const int col = tri_at(n, i + 1, i);   // packed index of A(i+1, i)
-        // xnorm^2 over A(i+2:n, i): per-thread partials, then thread 0 in order
-        double ss = 0.0;
-        for (int k = 1 + t; k < m; k += kTridThreads) ss += P[col + k] * P[col + k];
-        const double xn2 = tri_block_sum(ss, part);
-        if (t == 0) {
-            const double alpha = P[col];
-            if (xn2 == 0.0) {
-                sc[0] = 0.0; sc[1] = 1.0; sc[2] = alpha;
-            } else {
-                const double beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-                sc[0] = (beta - alpha) / beta;
-                sc[1] = 1.0 / (alpha - beta);
-                sc[2] = beta;
+    double dcur = A[0], ti = 0.0, beta = 0.0;
+    // stores step i; w = tau p + a2 v, x = row(i+1) - v(0) w - w(0) v below its
+    // diagonal and the next diagonal element
+    auto finish_step = [&](int i) {
+        const double *pb = ps[i & 1], *rb = rs[i & 1];
+        __syncthreads();
+        double p[NQ], r[NQ], pv[1] = {0.0};
+        const double p0 = pb[i + 1], r0 = rb[i + 1];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int c = ln + 64 * q;
+            p[q] = c > i && c < n ? pb[c] : 0.0;
+            r[q] = c > i && c < n ? rb[c] : 0.0;
+            pv[0] += p[q] * v[q];
+        }
+        if (wv == 0) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                const int c = ln + 64 * q;
+                if (c >= i && c < n) A[i * lda + c] = c == i ? dcur : c == i + 1 ? beta : v[q];
+            }
+            if (ln == 0) {
+                D[i] = dcur;
+                E[i] = beta;
+                tau[i] = ti;
             }
         }
-        __syncthreads();
-        const double ti = sc[0];
-        for (int k = t; k < m; k += kTridThreads)
-            v[k] = k == 0 ? 1.0 : (ti != 0.0 ? P[col + k] * sc[1] : P[col + k]);
-        __syncthreads();
-        if (ti != 0.0)
-            for (int k = 1 + t; k < m; k += kTridThreads) P[col + k] = v[k];
-        if (ti != 0.0) {
-            // w = tau A22 v over the symmetric trailing block (rows split into J chunks)
-            const int J = max(1, kTridThreads / m);
-            {
-                const int r = t / J, j = t - r * J;
-                double s2 = 0.0;
-                if (r < m)
-                    for (int c = j; c < m; c += J) {
-                        const int rr = max(r, c), cc = min(r, c);
-                        s2 += P[tri_at(n, i + 1 + rr, i + 1 + cc)] * v[c];
-                    }
-                part[t] = s2;
-            }
-            __syncthreads();
-            if (t < m) {
-                double s3 = 0.0;
-                for (int j = 0; j < J; j++) s3 += part[t * J + j];
-                w[t] = ti * s3;
-            }
-            __syncthreads();
-            // alpha2 = -tau/2 (w'v), w += alpha2 v
-            double dd = 0.0;
-            for (int k = t; k < m; k += kTridThreads) dd += w[k] * v[k];
-            const double s4 = tri_block_sum(dd, part);
-            if (t == 0) sc[3] = -0.5 * ti * s4;
-            __syncthreads();
-            for (int k = t; k < m; k += kTridThreads) w[k] += sc[3] * v[k];
-            __syncthreads();
-            // A22 -= v w' + w v' (lower triangle)
-            for (int e = t; e < m * m; e += kTridThreads) {
-                const int c = e / m, r = e - c * m;
-                if (r >= c) P[tri_at(n, i + 1 + r, i + 1 + c)] -= v[r] * w[c] + w[r] * v[c];
-            }
+        wave_sum_f64<1>(pv);
+        const double a2 = -0.5 * ti * (ti * pv[0]);
+        const double w0 = ti * p0 + a2;
+        dcur = r0 - (w0 + w0);
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            w[q] = ti * p[q] + a2 * v[q];
+            x[q] = ln + 64 * q > i + 1 ? r[q] - (w[q] + w0 * v[q]) : 0.0;
         }
-        __syncthreads();
-        if (t == 0) {
-            E[i] = sc[2];
-            D[i] = P[tri_at(n, i, i)];
-            tau[i] = ti;
-            P[col] = sc[2];
+    };
+#pragma unroll 1
+    for (int i = -1; i + 2 < n; i++) {
+        if (i >= 0) finish_step(i);
+        // dlarfg on x(i+2:n)
+        double vn[NQ], ss[1] = {0.0}, alpha = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int c = ln + 64 * q;
+            if (c > i + 2) ss[0] += x[q] * x[q];
+            if ((i + 2) >> 6 == q) alpha = readlane_f64(x[q], (i + 2) & 63);
         }
-        __syncthreads();
+        wave_sum_f64<1>(ss);
+        double scal = 1.0, tn = 0.0, bn = alpha;
+        if (ss[0] != 0.0) {
+            bn = -copysign(sqrt(alpha * alpha + ss[0]), alpha);
+            tn = (bn - alpha) / bn;
+            scal = 1.0 / (alpha - bn);
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int c = ln + 64 * q;
+            vn[q] = c == i + 2 ? 1.0 : tn != 0.0 ? x[q] * scal : x[q];
+        }
+        // rows i + 2 and below: A22 -= v w' + w v', and p = A22 v of the next step
+        double *pb = ps[(i + 1) & 1], *rb = rs[(i + 1) & 1];
+#pragma unroll
+        for (int k0 = 0; k0 < NK; k0 += 4) {
+            if (wv + kTridWaves * (k0 + 3) < i + 2 || wv + kTridWaves * k0 >= n) continue;
+            double s[4];
+#pragma unroll
+            for (int k = k0; k < k0 + 4; k++) {
+                const int r = wv + kTridWaves * k, rl = r & 63, rq = kTridWaves * k / 64;
+                const double vr = readlane_f64(v[rq], rl), wr = readlane_f64(w[rq], rl);
+                s[k - k0] = 0.0;
+#pragma unroll
+                for (int q = 0; q < NQ; q++) {
+                    a[k][q] = fma(-vr, w[q], fma(-wr, v[q], a[k][q]));
+                    s[k - k0] = fma(a[k][q], vn[q], s[k - k0]);
+                }
+                if (r == i + 2)
+#pragma unroll
+                    for (int q = 0; q < NQ; q++) rb[ln + 64 * q] = a[k][q];
+            }
+            const double t = rows4_sum(s[0], s[1], s[2], s[3]);
+            if ((ln & 15) == 0) pb[wv + kTridWaves * (k0 + (ln >> 4))] = t;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; q++) v[q] = vn[q];
+        ti = tn;
+        beta = bn;
     }
-    if (t == 0) {
-        D[n - 1] = P[tri_at(n, n - 1, n - 1)];
+    if (n > 1) finish_step(n - 2);
+    if (threadIdx.x == 0) {
+        D[n - 1] = dcur;
         tau[n - 1] = 0.0;
         E[n - 1] = 0.0;
-    }
-    __syncthreads();
-    for (int e = t; e < n * n; e += kTridThreads) {
-        const int c = e / n, r = e - c * n;
-        if (r >= c) A[(long)c * lda + r] = P[tri_at(n, r, c)];
+        A[(long)(n - 1) * lda + n - 1] = dcur;
     }
 }
 
 // The same reduction (dsytd2, UPLO = 'L', the same D, E, tau and vectors)
-// for matrices too large for one workgroup's LDS, in one cooperative launch
+// for matrices too large for one workgroup's registers, in one cooperative launch
 // of G workgroups.  Row r of the symmetric matrix lives in the LDS of
 // workgroup r mod G (both triangles, so the product A22 v is row-local).
 // Step i needs one grid barrier: before it every workgroup publishes its rows
@@ -1975,10 +1993,8 @@ int eigensolve_device(sgpu_context *ctx, int n, double *dA, double *dB, double *
         double *dtau = dE + n, *dC = dtau + n;
         SGPU_CHECK(sgpu_tbegin(ctx, &tp));
         if (lds) {
-            const size_t shm = ((size_t)n * (n + 1) / 2 + 2 * (size_t)n + kTridThreads) * sizeof(double);
-            SGPU_HIP(hipFuncSetAttribute((const void *)sytd2_lower_lds,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-            sytd2_lower_lds<<<1, kTridThreads, shm, ctx->stream>>>(dA, n, n, dD, dE, dtau);
+            auto kern = n <= 64 ? sytd2_lower_regs<1> : n <= 128 ? sytd2_lower_regs<2> : sytd2_lower_regs<3>;
+            kern<<<1, 64 * kTridWaves, 0, ctx->stream>>>(dA, n, n, dD, dE, dtau);
             SGPU_HIP(hipGetLastError());
         } else {
             if (ctx->coop_threads == 512)

@@ -198,6 +198,26 @@ def test_generalized_eigensolve_lds_tridiagonal(gpu, monkeypatch, n):
     assert np.max(np.abs(Q.T @ Hp @ Q - np.diag(lam))) < 1e-9
 
 
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 127, 128, 129, 179])
+def test_tridiagonal_in_registers_edges(gpu, n):
+    """The reduction in one workgroup's registers at the edges of its columns
+    per lane (64, 128) and with a last group of rows partly filled, on a
+    matrix with a zero column below the diagonal (tau = 0 in that step):
+    eigenvalues against LAPACK to 1e-10 and Mp-orthonormal eigenvectors, as in
+    test_generalized_eigensolve_lds_tridiagonal."""
+    from sparc_amd.workloads import Grid
+    rng = np.random.default_rng(170 + n)
+    F = rng.standard_normal((n, n))
+    Hp = (F + F.T) / 2 + np.diag(np.arange(n))
+    Hp[1:, 0] = Hp[0, 1:] = 0.0
+    Mp = np.eye(n)
+    with gpu.Context(Grid(8, 8, 8, 0.5, 0.5, 0.5)) as ctx:
+        lam, Q = ctx.DP_Solve_Generalized_EigenProblem(Hp, Mp)
+    assert np.max(np.abs(lam - sla.eigh(Hp, eigvals_only=True))) < 1e-10
+    assert np.max(np.abs(Q.T @ Q - np.eye(n))) < 1e-9
+    assert np.max(np.abs(Q.T @ Hp @ Q - np.diag(lam))) < 1e-9
+
+
 @pytest.mark.parametrize("ns", [24, 160, 300])
 def test_fp32_gram_accuracy(gpu, ns):
     """The FP32 projection (BF16-piece MFMA kernel below 256 states, rocBLAS
