@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "sgpu_internal.h"
+#include "wave_sum.h"
 
 namespace {
 
@@ -98,7 +99,10 @@ __global__ void aar_update_cols(double *xn, const double *x, const double *__res
 
 // The same sums as aar_gram for the columns F_j = f_(k-j) - f_(k-j-1), j < m.
 // Bound by reading m + 1 vectors; four workgroups per CU (with one, as
-// aar_gram has, too few bytes were in flight: 128^3, m = 7, 44 -> 33 us).
+// aar_gram has, too few bytes were in flight: 128^3, m = 7, 44 -> 38 us).  The
+// block's sums are taken four at a time with lane swaps (rows4_sum): 38 -> 23 us
+// there, 19.6 -> 5.3 us at 52^3, where the 35 butterflies of ds_bpermute were
+// most of the launch.
 template <int M>
 __global__ __launch_bounds__(256) void aar_gram_ring(AarRing f, int m, long n,
                                                      double *__restrict__ partial)
@@ -122,7 +126,17 @@ __global__ __launch_bounds__(256) void aar_gram_ring(AarRing f, int m, long n,
 #pragma unroll
         for (int a = 0; a < M; a++) acc[k++] += v[a] * fi;
     }
-    gram_partial<NV>(acc, partial);
+    __shared__ double sh[4][(NV + 3) / 4 * 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < NV; k += 4) {
+        const double s = rows4_sum(acc[k], k + 1 < NV ? acc[k + 1] : 0.0, k + 2 < NV ? acc[k + 2] : 0.0,
+                                   k + 3 < NV ? acc[k + 3] : 0.0);
+        if ((lane & 15) == 0) sh[wave][k + (lane >> 4)] = s;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < NV; k += 256)
+        partial[(long)blockIdx.x * NV + k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
 }
 
 // Partial sums of F'F (upper triangle, m(m+1)/2 values) and F'f (m values).
