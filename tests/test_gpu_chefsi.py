@@ -218,6 +218,30 @@ def test_tridiagonal_in_registers_edges(gpu, n):
     assert np.max(np.abs(Q.T @ Hp @ Q - np.diag(lam))) < 1e-9
 
 
+@pytest.mark.parametrize("n,groups", [(181, 32), (211, 7), (512, 32)])
+def test_tridiagonal_handover(gpu, monkeypatch, n, groups):
+    """Above 180 states the cooperative reduction hands the last 180 columns
+    to one workgroup (after its first step at n = 181, an owner of the next
+    row in mid-cycle with 7 groups): eigenvalues against LAPACK and the
+    reduction without the handover (SPARC_AMD_LDS_TRIDIAG=0) to 1e-10, and
+    eigenvectors that diagonalize Hp."""
+    from sparc_amd.workloads import Grid
+    rng = np.random.default_rng(190 + n)
+    F = rng.standard_normal((n, n))
+    Hp = (F + F.T) / 2
+    monkeypatch.setenv("SPARC_AMD_COOP_TRIDIAG", str(groups))
+    out = {}
+    for flag in ("1", "0"):
+        monkeypatch.setenv("SPARC_AMD_LDS_TRIDIAG", flag)
+        with gpu.Context(Grid(8, 8, 8, 0.5, 0.5, 0.5)) as ctx:
+            out[flag] = ctx.DP_Solve_Generalized_EigenProblem(Hp, np.eye(n))
+    lam, Q = out["1"]
+    assert np.max(np.abs(lam - sla.eigh(Hp, eigvals_only=True))) < 1e-10
+    assert np.max(np.abs(lam - out["0"][0])) < 1e-10
+    assert np.max(np.abs(Q.T @ Q - np.eye(n))) < 1e-9
+    assert np.max(np.abs(Q.T @ Hp @ Q - np.diag(lam))) < 1e-9
+
+
 @pytest.mark.parametrize("ns", [24, 160, 300])
 def test_fp32_gram_accuracy(gpu, ns):
     """The FP32 projection (BF16-piece MFMA kernel below 256 states, rocBLAS
