@@ -53,7 +53,7 @@ struct Mfma<float> {
     using acc = f32x4;
     using vec = float4;              // 16-byte staging vector
     static constexpr int NCP = 16;   // project: columns per block
-    static constexpr int NCA = 32;   // sphere apply: columns per block
+    static constexpr int NCA = 32;   // nlb_apply: columns per block
     static constexpr int NCB = 64;   // brick apply: columns per block
     __device__ static acc run(float a, float b, acc c)
     {
@@ -1628,7 +1628,6 @@ template <typename T>
 int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scale, T *alpha)
 {
     const sgpu_nonlocal &nl = ctx->nl;
-    constexpr int NCP = Mfma<T>::NCP;
     void *buf = nullptr;
     if (nl.mode == 1) {
         const int max_np = 64;
