@@ -82,7 +82,8 @@ int sgpu_set_veff(sgpu_context *ctx, const double *veff);
  * points grid_pos[pos_off[a]...], Chi as a column-major ndc[a] x nproj[a]
  * block at chi[chi_off[a]], and projector rows starting at alpha_off[a]
  * (IP_displ of its parent atom; images of one atom share rows).  gamma[r] is
- * Gamma_{l,p} of projector row r (n_alpha rows).  dV is the volume element. */
+ * Gamma_{l,p} of projector row r (n_alpha rows).  dV is the volume element.
+ * Entries with nproj[a] = 0 (local-only species) are checked and left out. */
 int sgpu_set_nonlocal(sgpu_context *ctx, int n_influence, const int *ndc, const int *nproj,
                       const long *pos_off, const int *grid_pos, const long *chi_off,
                       const double *chi, const int *alpha_off, int n_alpha,

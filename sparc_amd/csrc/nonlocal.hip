@@ -1629,6 +1629,9 @@ int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scal
 {
     const sgpu_nonlocal &nl = ctx->nl;
     void *buf = nullptr;
+    // rows that no entry has are zero
+    SGPU_HIP(hipMemsetAsync(alpha, 0, (size_t)nl.n_alpha * ncol * sizeof(T), ctx->stream));
+    if (nl.n_infl == 0) return SGPU_OK;
     if (nl.mode == 1) {
         const int max_np = 64;
         SGPU_CHECK(sgpu_scratch(ctx, (size_t)nl.n_ent * max_np * ncol * sizeof(T) + 256, &buf));
@@ -1736,46 +1739,66 @@ extern "C" int sgpu_nonlocal_integrals(sgpu_context *ctx, const sgpu_block *psi,
     return nonlocal_integrals_typed<float>(ctx, psi, out);
 }
 
-extern "C" int sgpu_set_nonlocal(sgpu_context *ctx, int n_influence, const int *ndc,
-                                 const int *nproj, const long *pos_off, const int *grid_pos,
-                                 const long *chi_off, const double *chi, const int *alpha_off,
-                                 int n_alpha, const double *gamma, double dV)
+extern "C" int sgpu_set_nonlocal(sgpu_context *ctx, int n_given, const int *ndc_given,
+                                 const int *nproj_given, const long *pos_off_given,
+                                 const int *grid_pos, const long *chi_off_given, const double *chi,
+                                 const int *alpha_off_given, int n_alpha, const double *gamma,
+                                 double dV)
 {
-    if (!ctx || n_influence < 0 || n_alpha < 0) {
+    if (!ctx || n_given < 0 || n_alpha < 0) {
         sgpu_set_error("sgpu_set_nonlocal: bad arguments");
         return SGPU_ERR_ARG;
     }
     SGPU_HIP(hipSetDevice(ctx->device));
     SGPU_HIP(hipStreamSynchronize(ctx->stream));
     sgpu_free_nonlocal(ctx->nl);
-    if (n_influence == 0 || n_alpha == 0) return SGPU_OK;
-    if (!ndc || !nproj || !pos_off || !grid_pos || !chi_off || !chi || !alpha_off || !gamma) {
+    if (n_given == 0 || n_alpha == 0) return SGPU_OK;
+    if (!ndc_given || !nproj_given || !pos_off_given || !grid_pos || !chi_off_given || !chi ||
+        !alpha_off_given || !gamma) {
         sgpu_set_error("sgpu_set_nonlocal: null array");
         return SGPU_ERR_ARG;
     }
+    // Entries without projectors (atoms of a local-only species) are checked
+    // like the others and then left out: they would make bricks of no rows,
+    // which nlb_chain's tiles do not provide for, and their alpha row is the
+    // next atom's, whose images they would join.
+    std::vector<int> ndc, nproj, alpha_off;
+    std::vector<long> pos_off, chi_off;
     const int nx = ctx->nx, ny = ctx->ny, nz = ctx->nz;
     const int nbx = (nx + kBX - 1) / kBX, nby = (ny + kBY - 1) / kBY, nbz = (nz + kBZ - 1) / kBZ;
     // (brick, entry) pairs, validated
     std::vector<std::pair<int, int>> pairs;
-    for (int a = 0; a < n_influence; a++) {
-        if (ndc[a] < 0 || nproj[a] < 0 || alpha_off[a] < 0 || alpha_off[a] + nproj[a] > n_alpha ||
-            pos_off[a] < 0 || chi_off[a] < 0) {
-            sgpu_set_error("sgpu_set_nonlocal: entry %d out of range", a);
+    for (int g = 0; g < n_given; g++) {
+        if (ndc_given[g] < 0 || nproj_given[g] < 0 || alpha_off_given[g] < 0 ||
+            alpha_off_given[g] + nproj_given[g] > n_alpha || pos_off_given[g] < 0 ||
+            chi_off_given[g] < 0) {
+            sgpu_set_error("sgpu_set_nonlocal: entry %d out of range", g);
             return SGPU_ERR_ARG;
         }
         std::vector<int> bl;
-        for (int i = 0; i < ndc[a]; i++) {
-            const int q = grid_pos[pos_off[a] + i];
+        for (int i = 0; i < ndc_given[g]; i++) {
+            const int q = grid_pos[pos_off_given[g] + i];
             if (q < 0 || q >= ctx->nd) {
-                sgpu_set_error("sgpu_set_nonlocal: grid_pos %d of entry %d outside the grid", q, a);
+                sgpu_set_error("sgpu_set_nonlocal: grid_pos %d of entry %d outside the grid", q, g);
                 return SGPU_ERR_ARG;
             }
             const int ix = q % nx, iy = (q / nx) % ny, iz = q / (nx * ny);
             bl.push_back((iz / kBZ * nby + iy / kBY) * nbx + ix / kBX);
         }
+        if (nproj_given[g] == 0) continue;
         std::sort(bl.begin(), bl.end());
         bl.erase(std::unique(bl.begin(), bl.end()), bl.end());
-        for (int b : bl) pairs.push_back({b, a});
+        for (int b : bl) pairs.push_back({b, (int)ndc.size()});
+        ndc.push_back(ndc_given[g]);
+        nproj.push_back(nproj_given[g]);
+        alpha_off.push_back(alpha_off_given[g]);
+        pos_off.push_back(pos_off_given[g]);
+        chi_off.push_back(chi_off_given[g]);
+    }
+    const int n_influence = (int)ndc.size();
+    if (n_influence == 0) {
+        ctx->nl.n_alpha = n_alpha;  // rows that the integrals report as zero
+        return SGPU_OK;
     }
     std::sort(pairs.begin(), pairs.end());
     {
@@ -1796,8 +1819,9 @@ extern "C" int sgpu_set_nonlocal(sgpu_context *ctx, int n_influence, const int *
         }
         if (np_max > 64) mode = 0;
         if (mode == 1)
-            return build_sphere_layout(ctx, n_influence, ndc, nproj, pos_off, grid_pos, chi_off, chi,
-                                       alpha_off, n_alpha, gamma, dV);
+            return build_sphere_layout(ctx, n_influence, ndc.data(), nproj.data(), pos_off.data(),
+                                       grid_pos, chi_off.data(), chi, alpha_off.data(), n_alpha, gamma,
+                                       dV);
     }
     // bricks, their column layout and row offsets
     std::vector<int> bid, borg, bnp;

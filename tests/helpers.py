@@ -48,6 +48,21 @@ def split_images(nl: NonlocalSet, entry: int = 0) -> NonlocalSet:
                        nl.n_alpha, nl.gamma.copy(), nl.dV)
 
 
+def with_bare_entries(nl: NonlocalSet, first, last) -> NonlocalSet:
+    """The same projectors with entries of no projectors (atoms of a local-only
+    species, on the given grid points) in front of and behind them; an entry's
+    alpha offset is the next atom's, n_alpha for the last one."""
+    k, pos = nl.n_influence, [np.asarray(p, np.int32) for p in (first, last)]
+    n0 = pos[0].size
+    return NonlocalSet(np.concatenate([[n0], nl.ndc, [pos[1].size]]).astype(np.int32),
+                       np.concatenate([[0], nl.nproj, [0]]).astype(np.int32),
+                       np.concatenate([[0], nl.pos_off + n0, [n0 + nl.grid_pos.size]]).astype(np.int64),
+                       np.concatenate([pos[0], nl.grid_pos, pos[1]]).astype(np.int32),
+                       np.concatenate([[0], nl.chi_off, [nl.chi.size]]).astype(np.int64), nl.chi,
+                       np.concatenate([nl.alpha_off[:1] if k else [0], nl.alpha_off, [nl.n_alpha]]).astype(np.int32),
+                       nl.n_alpha, nl.gamma, nl.dV)
+
+
 def rel_err(a, b):
     a = np.asarray(a)
     b = np.asarray(b)

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from tests.helpers import rel_err, small_case, split_images
+from tests.helpers import rel_err, small_case, split_images, with_bare_entries
 
 pytestmark = pytest.mark.gpu
 
@@ -292,3 +292,46 @@ def test_vnl_psp_projectors(gpu, oracle_mod, nl_mode, mode):
     assert rel_err(y, yo) < 1e-12
     x32 = x.astype(np.float32).astype(np.float64)
     assert rel_err(y32, o.hamiltonian(x32)) < 2e-6
+
+
+@pytest.mark.parametrize("mode", ["brick", "sphere"])
+def test_entries_without_projectors(gpu, nl_mode, mode):
+    """Atoms without projectors, first and last in the list and alone in the
+    grid's first and last brick, change nothing: apply, filter (the fused
+    chain) and integrals are bitwise those of the set without them."""
+    nl_mode(mode)
+    g, veff, nl, rng = small_case(n=(36, 18, 12), n_sites=1, rc=1.2, seed=17)
+    bricks = [(i % 36 // 16, i // 36 % 18 // 8, i // (36 * 18) // 4) for i in range(g.nd)]
+    taken = {bricks[i] for i in nl.grid_pos}
+    free = sorted(set(bricks) - taken)
+    assert (0, 0, 0) in free and (2, 2, 2) in free  # the bare atoms' bricks hold no other entry
+    bare = with_bare_entries(nl, [i for i in range(g.nd) if bricks[i] == (0, 0, 0)][:100],
+                             [i for i in range(g.nd) if bricks[i] == (2, 2, 2)])
+    x = rng.uniform(-0.5, 0.5, (g.nd, 21))
+    for dt in (gpu.F64, gpu.F32):
+        outs = []
+        for s in (nl, bare):
+            with gpu.Context(g) as ctx:
+                ctx.set_veff(veff)
+                ctx.set_nonlocal(s)
+                bx, by = ctx.block(21, dt).upload(x), ctx.block(21, dt)
+                ctx.hamiltonian_dev(0.2, bx, by)
+                o = [by.download(), ctx.nonlocal_integrals(bx)]
+                ctx.chebyshev_filter_dev(bx, by, 4, 2.0, 90.0, -3.0)
+                outs.append(o + [by.download(), bx.download()])
+        for a, b in zip(*outs):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+def test_only_entries_without_projectors(gpu):
+    """A set of bare atoms alone acts as no projectors; its rows' integrals are zero."""
+    g, veff, nl, rng = small_case(n=(20, 18, 16), seed=18)
+    only = with_bare_entries(type(nl)(nl.ndc[:0], nl.nproj[:0], nl.pos_off[:0], nl.grid_pos[:0], nl.chi_off[:0],
+                                      nl.chi[:1], nl.alpha_off[:0], nl.n_alpha, nl.gamma, nl.dV), [5, 6, 7], [9])
+    x = rng.uniform(-0.5, 0.5, (g.nd, 3))
+    with gpu.Context(g) as ctx:
+        ctx.set_veff(veff)
+        y = ctx.Hamiltonian_vectors_mult(x, 0.2)
+        ctx.set_nonlocal(only)
+        assert np.array_equal(ctx.Hamiltonian_vectors_mult(x, 0.2), y)
+        assert not ctx.nonlocal_integrals(ctx.block(3, gpu.F64).upload(x)).any()
