@@ -88,22 +88,30 @@ int apply_h_chain(sgpu_context *ctx, int dtype, int ncol, double c, const void *
 }
 
 // Columns that a filter takes at a time: with the sphere layout in one colour,
-// panels whose two buffers stay in the 256 MB Infinity Cache over all degrees
-// (at most 96 MB each, equal, in multiples of 8), where the block itself is too
-// large for that.  Degree 20: 78^3 x 480 FP32, 216 atoms, 23.4 -> 19.3 ms (10
-// panels of 48; of 64, 121 MB, 20.7, of 32 22.5), 64 atoms 17.3 -> 14.7; 96^3 x
-// 256 FP32, 216 atoms, 19.0 -> 15.3; 52^3 x 160 FP64, 64 atoms, 3.82 -> 3.40;
-// 78^3 x 72 FP32 (137 MB) 3.41 -> 3.25, but x 64 (121 MB) in halves 2.81 ->
-// 2.87.  With fewer than 128 blocks in the nonlocal launches (52^3 x 170 FP64,
-// 8 atoms: 2.94 -> 3.15) or in several colours (40^3 x 512 FP64, 27 atoms: 6.5
-// -> 7.3) the shorter launches cost more than the cache gives; so do they in
-// the brick layout, whose blocks take 128 columns (96^3 x 512: 59 -> 62).
+// equal panels, in multiples of 8 columns, whose two buffers stay in the 256 MB
+// Infinity Cache over all degrees (at most 96 MB each, after the rounding),
+// where the block itself is too large for that.  Degree 20, whole block ->
+// panels, 8 projectors an atom: 78^3 x 480 FP32, 216 atoms, 23.4 -> 19.3 ms (10
+// panels of 48; of 64, 121 MB, 20.7, of 32 22.5); 88^3 x 300 FP32 20.4 -> 16.4
+// (of 32; of 40, 109 MB, 17.9); 52^3 x 160 FP64, 64 atoms, 3.82 -> 3.40; 70^3 x
+// 200 FP64 12.1 -> 10.4 (of 32; of 40, 110 MB, 11.4); 87^3 x 200 FP64 24.1 ->
+// 20.8 (of 16; of 24, 126 MB, 27.4).  78^3 x 72 FP32 (137 MB) 3.41 -> 3.25, but
+// x 64 (121 MB) in halves 2.81 -> 2.87.  With 18 projectors (two row tiles) 88^3
+// x 300 FP32 20.9 -> 17.1 and 70^3 x 200 FP64 12.5 -> 11.5, but panels below 32
+// columns give nothing: 78^3 x 200 FP64 17.5 -> 17.7 (of 24), 100^3 x 300 FP32
+// 29.1 -> 30.6 (of 24), 87^3 x 200 FP64 24.5 -> 28.7 (of 16).  With fewer than
+// 128 blocks in the nonlocal launches (52^3 x 170 FP64, 8 atoms: 2.94 -> 3.15)
+// or in several colours (40^3 x 512 FP64, 27 atoms: 6.5 -> 7.3) the shorter
+// launches cost more than the cache gives; so do they in the brick layout, whose
+// blocks take 128 columns (96^3 x 512: 59 -> 62).
 int filter_panel(sgpu_context *ctx, int dtype, int ncol)
 {
     const sgpu_nonlocal &nl = ctx->nl;
-    const double bytes = (double)ctx->nd * ncol * (dtype == SGPU_F64 ? 8 : 4);
-    if (nl.mode != 1 || nl.n_colors != 1 || !ctx->nl_chain || bytes < 136e6) return ncol;
-    const int np = (int)(bytes / 96e6) + 1;
+    const double col = (double)ctx->nd * (dtype == SGPU_F64 ? 8 : 4);
+    if (nl.mode != 1 || nl.n_colors != 1 || !ctx->nl_chain || col * ncol < 136e6) return ncol;
+    const int most = (int)std::min(96e6 / col, 1e6) / 8 * 8;
+    if (most < (nl.max_npad > 16 ? 32 : 16)) return ncol;
+    const int np = (ncol + most - 1) / most;
     const int panel = ((ncol + np - 1) / np + 7) / 8 * 8;
     return (long)nl.n_ent * ((panel + 15) / 16) < 128 ? ncol : std::min(panel, ncol);
 }

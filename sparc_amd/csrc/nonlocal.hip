@@ -931,11 +931,20 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 2) void nlb_chain(
 // column panels).  In three colours, 45 x 51 x 73 x 37 FP64: 10.5 against
 // 17.5 us a colour, the projection 8.5 against 22 us.
 constexpr int kEnt = 8;            // ints per entry in ent_info
-// Waves per block.  16 rather than 8, 12 or 4 where one projector tile leaves
-// the registers (at most 128): a whole entry is then one or two groups of
-// loads.  26^3 x 24 FP32, 8 atoms, per launch: 8.5 us, against 13.0 us with 8
-// waves.
-constexpr int nls_waves(int rt) { return rt == 1 ? 16 : 8; }
+// Waves per block, by row tiles and the launch's blocks.  One tile leaves the
+// registers for 16 (at most 128): a whole entry is then one or two groups of
+// loads (26^3 x 24 FP32, 8 atoms, per launch: 8.5 us, against 13.0 us with 8
+// waves).  With more tiles 8; but of the FP64 form with two tiles (134 to 140
+// registers, three waves a SIMD) a CU holds one block of 8 waves or three of 4,
+// so a launch of more blocks than CUs takes 4: 78^3 x 480 with 18 projectors an
+// atom 749 -> 665 us, in panels of 80 columns of 52^3 (320 blocks) 39.1 -> 34.4,
+// while 256 blocks (64 columns) take 24.2 us with 8 waves and 28.7 with 4.  In
+// FP32 (122 registers, two blocks of 8) 8 and 4 are within 5 % either way.
+template <typename T>
+constexpr int nls_waves(int rt, bool many)
+{
+    return rt == 1 ? 16 : rt == 2 && many && sizeof(T) == 8 ? 4 : 8;
+}
 
 // Orders a wavefront's LDS writes before its later LDS reads and the reads
 // before later writes, for data exchanged between lanes of one wave only:
@@ -948,10 +957,10 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// RT: 16-row projector tiles (npad <= 16 RT); APPLY / PROJ as above (out is
-// only read without APPLY).
-template <typename T, int RT, bool APPLY, bool PROJ>
-__global__ __launch_bounds__(64 * nls_waves(RT)) void nls_chain(
+// RT: 16-row projector tiles (npad <= 16 RT); NW: waves; APPLY / PROJ as above
+// (out is only read without APPLY).
+template <typename T, int RT, int NW, bool APPLY, bool PROJ>
+__global__ __launch_bounds__(64 * NW) void nls_chain(
     T *out, long ldo, int ncol, int e0, const int *__restrict__ ent_info,
     const long *__restrict__ ent_chi, const int *__restrict__ gpos, const T *__restrict__ chir,
     const T *__restrict__ chit, const int *__restrict__ atom_img, const double *__restrict__ gamma,
@@ -959,7 +968,7 @@ __global__ __launch_bounds__(64 * nls_waves(RT)) void nls_chain(
 {
     using M = Mfma<T>;
     using acc_t = typename M::acc;
-    constexpr int NW = nls_waves(RT), GT = sizeof(T) == 8 || RT > 2 ? 1 : RT == 2 ? 2 : 3, LDY = 17;
+    constexpr int GT = sizeof(T) == 8 || RT > 2 ? 1 : RT == 2 ? 2 : 3, LDY = 17;
     __shared__ T ytile[PROJ ? NW * 16 * LDY : 1];
     __shared__ acc_t red[PROJ ? NW * RT : 1][64];
     // the column blocks of one entry are consecutive logical ids -> one XCD
@@ -1092,14 +1101,17 @@ int launch_nls(sgpu_context *ctx, int ncol, T *out, long ldo, int e0, int ne, co
 {
     const sgpu_nonlocal &nl = ctx->nl;
     const dim3 grid((ncol + 15) / 16, ne);
-    auto go = [&](auto kern, int waves) {
-        kern<<<grid, 64 * waves, 0, ctx->stream>>>(out, ldo, ncol, e0, nl.ent_info, nl.ent_chi, nl.gpos,
-                                                       chir, chit, nl.atom_img, nl.gamma, scale_dv, part,
-                                                       64, part_next);
+    auto go = [&](auto rt, auto many) {
+        constexpr int RT = decltype(rt)::value, NW = nls_waves<T>(RT, decltype(many)::value);
+        nls_chain<T, RT, NW, APPLY, PROJ><<<grid, 64 * NW, 0, ctx->stream>>>(
+            out, ldo, ncol, e0, nl.ent_info, nl.ent_chi, nl.gpos, chir, chit, nl.atom_img, nl.gamma,
+            scale_dv, part, 64, part_next);
     };
-    if (nl.max_npad <= 16) go(nls_chain<T, 1, APPLY, PROJ>, nls_waves(1));
-    else if (nl.max_npad <= 32) go(nls_chain<T, 2, APPLY, PROJ>, nls_waves(2));
-    else go(nls_chain<T, 4, APPLY, PROJ>, nls_waves(4));
+    using std::integral_constant;
+    if (nl.max_npad <= 16) go(integral_constant<int, 1>{}, std::false_type{});
+    else if (nl.max_npad > 32) go(integral_constant<int, 4>{}, std::false_type{});
+    else if ((long)grid.x * ne > ctx->n_cu) go(integral_constant<int, 2>{}, std::true_type{});
+    else go(integral_constant<int, 2>{}, std::false_type{});
     SGPU_HIP(hipGetLastError());
     return SGPU_OK;
 }

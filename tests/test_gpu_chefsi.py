@@ -445,6 +445,51 @@ def test_filter_column_panels(gpu, oracle_mod, monkeypatch, dtype, ncol, m):
         assert rel_err(whole[:, cols], part) < (1e-13 if dtype == 0 else 1e-5)
 
 
+def test_filter_panels_fit_the_cache(gpu, monkeypatch):
+    """341 FP32 columns of 52^3 in panels of at most 96 MB (170 columns) after
+    the rounding to 8 columns: three panels, each with its own first projection
+    (in two, of 176 columns, they would be 99 MB)."""
+    from sparc_amd.workloads import Grid, gaussian_projectors
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "sphere")
+    g = Grid(52, 52, 52, 0.5, 0.5, 0.5)
+    c = np.arange(4) * 6.5 + 3.0
+    sites = np.stack(np.meshgrid(c, c, c, indexing="ij"), -1).reshape(-1, 3)
+    with gpu.Context(g) as ctx:
+        ctx.set_veff(np.zeros(g.nd))
+        ctx.set_nonlocal(gaussian_projectors(g, sites, 1.6, sigmas=(1.0,), gammas=(1.3,), lmax=1))
+        bx = ctx.block(341, gpu.F32).fill_uniform(3, -0.5, 0.5)
+        ctx.timer_enable(True)
+        ctx.chebyshev_filter_dev(bx, ctx.block(341, gpu.F32), 2, 2.0, 60.0, -1.0)
+        assert ctx.timer("nl_project")[1] == 3
+
+
+def test_sphere_chain_many_blocks(gpu, monkeypatch):
+    """FP64 with two row tiles and more blocks than CUs (4 entries x 66 column
+    blocks: four waves a block instead of eight): the fused filter bitwise the
+    unfused one, and its columns those of a narrow block (eight waves) but for
+    the order of the waves' sums over 4 applications, 1e-13."""
+    from sparc_amd.workloads import Grid, gaussian_projectors, gaussian_veff
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "sphere")
+    g = Grid(21, 20, 18, 0.5, 0.5, 0.5)
+    rng = np.random.default_rng(73)
+    veff = gaussian_veff(g, 4, rng)
+    sites = np.array([[2.5, 7.5, 6.5], [7.6, 2.5, 2.5], [0.2, 2.5, 7.0], [5.2, 5.2, 0.2]])
+    nl = gaussian_projectors(g, sites, 1.5, sigmas=(0.8, 0.5), gammas=(1.3, -0.6), lmax=2)
+    ncol = 1050
+    out = []
+    for chain, cols in (("1", slice(0, ncol)), ("0", slice(0, ncol)), ("1", slice(1030, ncol))):
+        monkeypatch.setenv("SPARC_AMD_NL_CHAIN", chain)
+        with gpu.Context(g) as ctx:
+            ctx.set_veff(veff)
+            ctx.set_nonlocal(nl)
+            X = np.random.default_rng(74).uniform(-0.5, 0.5, (g.nd, ncol))[:, cols]
+            bx, by = ctx.block(X.shape[1], gpu.F64).upload(X), ctx.block(X.shape[1], gpu.F64)
+            ctx.chebyshev_filter_dev(bx, by, 4, 2.0, 60.0, -1.0)
+            out.append(by.download())
+    assert np.array_equal(out[0], out[1])
+    assert rel_err(out[0][:, 1030:], out[2]) < 1e-13
+
+
 @pytest.mark.parametrize("n,groups,threads", [(181, 32, 256), (300, 7, 256), (480, 32, 256),
                                               (480, 64, 512), (1000, 16, 256)])
 def test_generalized_eigensolve_cooperative_tridiagonal(gpu, monkeypatch, n, groups, threads):
