@@ -17,9 +17,10 @@
 //     next step's partials from the updated values (SPARC_AMD_NL_CHAIN_BRICK=0
 //     keeps them apart), so 1. runs once per filter.
 //
-// Bricks of more than 112 rows take nlb_project_rs (X streamed straight into
-// the MFMA operands, the four wavefronts splitting the brick's points) and
-// nlb_apply_rs (beta in LDS).
+// Narrow blocks of columns (nlb_chain_takes), and layouts in which any brick has
+// more than 112 rows, take nlb_project_rs (X streamed straight into the MFMA
+// operands, the four wavefronts splitting the brick's points) and nlb_apply_rs
+// (beta in LDS), unfused.
 // The LDS-staged forms (nlb_project, 16 columns per block; the transposed
 // nlb_apply, 32 columns) stay selectable with SPARC_AMD_NLB=lds.  On the
 // 96^3 x 512 FP32 operator case: 1.04 -> 0.74 ms (projection) and
@@ -521,8 +522,8 @@ __global__ __launch_bounds__(256) void nlb_apply(T *__restrict__ out, long ldo, 
 // covering 16 columns' 64-byte (128-byte) segments of the row, and the A
 // operand (Phi_b column-major, points contiguous) is a coalesced load shared
 // by the NC / 16 column tiles.
-// Every lane's loads of a row step are issued before its MFMAs.  Taken by bricks
-// of more rows than nlb_chain holds.
+// Every lane's loads of a row step are issued before its MFMAs.  Taken where
+// nlb_chain_takes says no.
 template <typename T, int NC>
 __global__ __launch_bounds__(256) void nlb_apply_rs(T *__restrict__ out, long ldo, int ncol, int nx,
                                                     int ny, int nz, const int *__restrict__ brick_org,
@@ -1127,13 +1128,36 @@ bool nlb_lds_kernels()
     return v;
 }
 
-// Whether nlb_chain takes the layout: its register tiles hold the bricks' rows
-// and 16 columns stay below 2^31 bytes.
+// What a launch over the bricks is part of: a projection or an apply by itself,
+// or a filter, whose applies also form the next projection.
+enum class NlbPass { Project, Apply, Filter };
+
+// Whether nlb_chain takes the launch: its register tiles hold every brick's
+// rows, 16 columns stay below 2^31 bytes, and its 128-column blocks have enough
+// columns for their waves (a wave without columns waits for the others, which
+// each walk the whole brick), against nlb_project_rs and nlb_apply_rs, where
+// four waves share 16 to 64 columns.  96^3, 64 sites of 6 Bohr, us per launch,
+// rs -> nlb_chain.  Filter, per degree (both rs launches against the fused one):
+// FP32 x 1 242 -> 274, x 48 295 -> 299, x 56 314 -> 303, x 96 497 -> 327, x 144
+// 682 -> 571; FP64 x 1 266 -> 598, x 32 393 -> 612, x 56 610 -> 627, x 64 630 ->
+// 633, x 72 778 -> 640, x 144 1353 -> 1211.  Projection: FP32 x 64 118 -> 150,
+// x 72 181 -> 152, x 144 261 -> 272, x 192 279 -> 275; FP64 x 64 284 -> 347, x 72
+// 382 -> 351, x 144 641 -> 638.  Apply: FP32 x 64 183 -> 188, x 72 272 -> 192, x
+// 144 385 -> 428, x 192 447 -> 456, x 200 551 -> 455; FP64 x 96 452 -> 495, x 128
+// 600 -> 540, x 192 857 -> 1012, x 200 955 -> 1030, x 256 1187 -> 1057.
+// SPARC_AMD_NLB=chain takes every width.
 template <typename T>
-bool nlb_chain_fits(const sgpu_context *ctx, long ldo)
+bool nlb_chain_takes(const sgpu_context *ctx, long ldo, int ncol, NlbPass pass)
 {
-    return !nlb_lds_kernels() && ctx->nl.max_np <= 16 * Chain<T>::RTM &&
-           16 * ldo * (long)sizeof(T) < 0x7ffffff0L;
+    if (nlb_lds_kernels() || ctx->nl.max_np > 16 * Chain<T>::RTM ||
+        16 * ldo * (long)sizeof(T) >= 0x7ffffff0L)
+        return false;
+    if (ctx->nlb_any_width) return true;
+    constexpr bool F32 = sizeof(T) == 4;
+    if (pass == NlbPass::Filter) return ncol >= (F32 ? 52 : 64);
+    if (pass == NlbPass::Project) return ncol > 64;
+    const int blocks = (ncol + Chain<T>::NC - 1) / Chain<T>::NC;
+    return F32 ? ncol > 64 && (blocks != 2 || ncol > 192) : 8 * ncol >= 7 * Chain<T>::NC * blocks;
 }
 
 template <typename T, bool APPLY, bool PROJ>
@@ -1162,7 +1186,7 @@ int launch_nlb_chain(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi
 // partials Phi_b' out of the result.
 template <typename T>
 int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phic, const T *alpha_s,
-                     T *part_next)
+                     T *part_next, NlbPass pass)
 {
     const sgpu_nonlocal &nl = ctx->nl;
     if (nlb_lds_kernels() && !part_next) {
@@ -1178,7 +1202,7 @@ int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi
             nl.row_alpha, phic, alpha_s);
         return SGPU_OK;
     }
-    if (nlb_chain_fits<T>(ctx, ldo)) {
+    if (nlb_chain_takes<T>(ctx, ldo, ncol, pass)) {
         if (part_next)
             return launch_nlb_chain<T, true, true>(ctx, ncol, out, ldo, phic, alpha_s, part_next);
         return launch_nlb_chain<T, true, false>(ctx, ncol, out, ldo, phic, alpha_s, nullptr);
@@ -1203,15 +1227,15 @@ int launch_nlb_apply(sgpu_context *ctx, int ncol, T *out, long ldo, const T *phi
     return go(nlb_apply_rs<T, NC>);
 }
 
-// part = Phi_b' X for every brick: nlb_project_rs with 64 (FP32) / 32 (FP64)
-// columns per block, 16-byte loads where the grid and X allow them.
+// part = Phi_b' X for every brick: nlb_chain, or nlb_project_rs with 64 (FP32) /
+// 32 (FP64) columns per block, 16-byte loads where the grid and X allow them.
 template <typename T>
 int launch_nlb_project(sgpu_context *ctx, int ncol, const T *x, long ldx, const T *phi, const T *phic,
-                       T *part)
+                       T *part, NlbPass pass)
 {
     const sgpu_nonlocal &nl = ctx->nl;
     const hipStream_t stream = ctx->stream;
-    if (nlb_chain_fits<T>(ctx, ldx))
+    if (nlb_chain_takes<T>(ctx, ldx, ncol, pass))
         return launch_nlb_chain<T, false, true>(ctx, ncol, const_cast<T *>(x), ldx, phic, nullptr, part);
     if (nlb_lds_kernels()) {
         constexpr int NCP = Mfma<T>::NCP;
@@ -1276,7 +1300,8 @@ int launch_vnl_sphere(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out,
 
 template <typename T>
 int launch_vnl_typed(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, long ldo,
-                     double scale, const T *phi, const T *phic, void *ws, size_t ws_bytes)
+                     double scale, const T *phi, const T *phic, void *ws, size_t ws_bytes,
+                     bool filter = false)
 {
     const sgpu_nonlocal &nl = ctx->nl;
     if (nl.n_bricks == 0 || nl.n_alpha == 0 || ncol <= 0) return SGPU_OK;
@@ -1291,7 +1316,8 @@ int launch_vnl_typed(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, 
     T *alpha_s = part + part_elems;
     sgpu_tmark t;
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part));
+    SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part,
+                                     filter ? NlbPass::Filter : NlbPass::Project));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     const long total = (long)nl.n_alpha * ncol;
@@ -1299,7 +1325,8 @@ int launch_vnl_typed(sgpu_context *ctx, int ncol, const T *x, long ldx, T *out, 
         part, ncol, nl.n_alpha, nl.arow_ptr, nl.arow_src, nl.gamma, scale * nl.dV, alpha_s);
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s, nullptr));
+    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s, nullptr,
+                                   filter ? NlbPass::Filter : NlbPass::Apply));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
     return SGPU_OK;
@@ -1381,9 +1408,10 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
         sgpu_set_error("nonlocal: %d bricks exceed the launch limit", nl.n_bricks);
         return SGPU_ERR_ARG;
     }
-    const bool fuse = want_next && ctx->nl_chain_brick && nlb_chain_fits<T>(ctx, ldo);
+    const bool fuse =
+        want_next && ctx->nl_chain_brick && nlb_chain_takes<T>(ctx, ldo, ncol, NlbPass::Filter);
     if (!fuse && !have_part)
-        return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0);
+        return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0, true);
     const size_t part_elems = (size_t)nl.n_rows * ncol;
     const size_t need = (2 * part_elems + (size_t)nl.n_alpha * ncol) * sizeof(T) + 256;
     if (have_part && need > nl.chain_bytes) {
@@ -1394,7 +1422,7 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
     if (chain_buffer(ctx, need, &buf) < 0) {
         // no room for two sets of partials: the separate launches need one
         (void)hipGetLastError();
-        return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0);
+        return launch_vnl_typed<T>(ctx, ncol, x, ldx, out, ldo, scale, phi, phic, nullptr, 0, true);
     }
     if (!have_part) nl.chain_cur = 0;
     T *part = (T *)buf + (size_t)nl.chain_cur * part_elems;
@@ -1403,7 +1431,7 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
     sgpu_tmark t;
     if (!have_part) {
         SGPU_CHECK(sgpu_tbegin(ctx, &t));
-        SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part));
+        SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx, phi, phic, part, NlbPass::Filter));
         SGPU_HIP(hipGetLastError());
         SGPU_CHECK(sgpu_tend(ctx, &t, "nl_project"));
     }
@@ -1412,8 +1440,8 @@ int launch_vnl_chain_brick(sgpu_context *ctx, int ncol, const T *x, long ldx, T 
         part, ncol, nl.n_alpha, nl.arow_ptr, nl.arow_src, nl.gamma, scale * nl.dV, alpha_s);
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tbegin(ctx, &t));
-    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s,
-                                   fuse ? part_next : nullptr));
+    SGPU_CHECK(launch_nlb_apply<T>(ctx, ncol, out, ldo, phic, alpha_s, fuse ? part_next : nullptr,
+                                   NlbPass::Filter));
     SGPU_HIP(hipGetLastError());
     SGPU_CHECK(sgpu_tend(ctx, &t, "nl_apply"));
     if (fuse) {
@@ -1667,7 +1695,7 @@ int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scal
         SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx,
                                          sizeof(T) == 8 ? (const T *)nl.phi64 : (const T *)nl.phi32,
                                          sizeof(T) == 8 ? (const T *)nl.phic64 : (const T *)nl.phic32,
-                                         part));
+                                         part, NlbPass::Project));
         SGPU_HIP(hipGetLastError());
         const long total = (long)nl.n_alpha * ncol;
         nlb_reduce<T><<<(unsigned)((total + 255) / 256), 256, 0, ctx->stream>>>(

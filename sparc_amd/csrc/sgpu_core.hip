@@ -73,6 +73,7 @@ extern "C" int sgpu_create(sgpu_context **out, int device, int nx, int ny, int n
     if (const char *t = getenv("SPARC_AMD_STENCIL_TILE")) ctx->stencil_cfg = atoi(t);
     if (const char *t = getenv("SPARC_AMD_NL_CHAIN")) ctx->nl_chain = atoi(t) != 0;
     if (const char *t = getenv("SPARC_AMD_NL_CHAIN_BRICK")) ctx->nl_chain_brick = atoi(t) != 0;
+    if (const char *t = getenv("SPARC_AMD_NLB")) ctx->nlb_any_width = strcmp(t, "chain") == 0;
     if (const char *t = getenv("SPARC_AMD_LDS_TRIDIAG")) ctx->lds_tridiag = atoi(t) != 0;
     if (const char *t = getenv("SPARC_AMD_COOP_TRIDIAG")) ctx->coop_tridiag = std::max(0, atoi(t));
     if (const char *t = getenv("SPARC_AMD_COOP_THREADS")) ctx->coop_threads = atoi(t) == 512 ? 512 : 256;

@@ -146,6 +146,9 @@ struct sgpu_context {
     // turns it off): 96^3 x 512 FP32 1.14 ms per application against 1.01 +
     // 0.57 ms for the apply and the projection apart, bitwise equal
     bool nl_chain_brick = true;
+    // nlb_chain for any number of columns (SPARC_AMD_NLB=chain; by default
+    // narrow blocks take the launches whose waves share their columns)
+    bool nlb_any_width = false;
     // eigensolves of up to 180 states reduce to tridiagonal form in one
     // workgroup's LDS instead of rocsolver's dsytrd (SPARC_AMD_LDS_TRIDIAG=0
     // keeps dsyevd everywhere)

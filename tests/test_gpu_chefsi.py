@@ -372,6 +372,45 @@ def test_brick_chain_edges(gpu, oracle_mod, monkeypatch, n, sites, lmax, ncol, d
 
 
 @pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("n,sites,lmax,ncol", [
+    ((20, 18, 16), 1, 0, 1),      # two rows: one tile, one column of 128
+    ((21, 17, 16), 4, 1, 17),     # 32 rows, two waves with columns, x-rows ending inside a lane's points
+    ((34, 20, 17), 5, 2, 16),     # 72 rows (five tiles, the last partly filled), one wave with columns
+    ((24, 20, 17), 4, 1, 145),    # a second block with two waves' columns
+])
+def test_brick_chain_any_width(gpu, oracle_mod, monkeypatch, n, sites, lmax, ncol, dtype):
+    """nlb_chain with waves that have no columns, which its rule leaves to
+    other kernels (SPARC_AMD_NLB=chain takes every width)."""
+    monkeypatch.setenv("SPARC_AMD_NLB", "chain")
+    test_brick_chain_edges(gpu, oracle_mod, monkeypatch, n, sites, lmax, ncol, dtype)
+
+
+@pytest.mark.parametrize("dtype,ncol,fused", [(1, 1, False), (1, 51, False), (1, 52, True), (1, 129, True),
+                                              (0, 1, False), (0, 63, False), (0, 64, True)])
+def test_brick_chain_width_rule(gpu, oracle_mod, monkeypatch, dtype, ncol, fused):
+    """Blocks of few columns are filtered with the launches whose waves share
+    them (a projection per degree), wider ones with the fused pass (one in all);
+    one application, projection included, on both sides against the oracle.
+    Tolerances as in test_filter_nonlocal_chain, and of test_vnl_fp64 /
+    test_hamiltonian_fp32_block for the application."""
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "brick")
+    g, veff, nl, rng = small_case(n=(21, 18, 17), n_sites=4, rc=3.2, seed=62, lmax=1)
+    o = oracle_mod.Oracle(g, veff, nl)
+    a0, b, a = _bounds(o, g)
+    X = rng.uniform(-0.5, 0.5, (g.nd, ncol)).astype(np.float32).astype(np.float64)
+    with gpu.Context(g) as ctx:
+        ctx.set_veff(veff)
+        ctx.set_nonlocal(nl)
+        bx, by = ctx.block(ncol, dtype).upload(X), ctx.block(ncol, dtype)
+        ctx.hamiltonian_dev(0.1, bx, by)
+        assert rel_err(by.download(), o.hamiltonian(X, 0.1)) < (1e-12 if dtype == 0 else 2e-6)
+        ctx.timer_enable(True)
+        ctx.chebyshev_filter_dev(bx, by, 4, a, b, a0)
+        assert ctx.timer("nl_project")[1] == (1 if fused else 4)
+        assert rel_err(by.download(), o.chebyshev_filter(X, 4, a, b, a0)[0]) < (1e-11 if dtype == 0 else 1e-4)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("rc,lmax,nsig,ncol", [
     (0.6, 0, 1, 1),     # a handful of points, one row, one column
     (2.4, 1, 2, 17),    # 8 rows, more point tiles than waves
