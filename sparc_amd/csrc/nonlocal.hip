@@ -705,7 +705,9 @@ __device__ __forceinline__ void nlb_chain_brick(
     constexpr int VW = 16 / sizeof(T), NV = 4 / VW, SZ = sizeof(T);
     constexpr int CH = K::CH, LDP = K::LDP, NS = CH / 16;  // NS x-rows per chunk
     constexpr int BUF = 16 * RT * LDP;
-    constexpr int kOff = 0x7ffffff0;  // past every resource: reads zero, stores nothing
+    // past every resource: reads zero, stores nothing (offsets are unsigned: its
+    // sums with a row's offset and a piece's pass 2^31)
+    constexpr unsigned kOff = 0x7ffffff0;
     const int x0 = brick_org[3 * b], y0 = brick_org[3 * b + 1], z0 = brick_org[3 * b + 2];
     const long row0 = brick_row[b];
     const T *pc = phic + row0 * kBP;
@@ -721,32 +723,31 @@ __device__ __forceinline__ void nlb_chain_brick(
     const bool cok = li < nc;
     // lane part of the offset of my four points (element e for !VEC)
     const int xl = x0 + 4 * lk;
-    const int vo = cok && xl < nx ? (int)((li * ldo + xl) * SZ) : kOff;
+    const unsigned vo = cok && xl < nx ? (unsigned)((li * ldo + xl) * SZ) : kOff;
     auto row_off = [&](int step) {  // byte offset of x-row `step` of the brick, -1: outside
         const int y = y0 + step % kBY, z = z0 + step / kBY;
         return y < ny && z < nz ? (z * ny + y) * nx * SZ : -1;
     };
     auto load4 = [&](int step, T (&v)[4]) {
         const int ro = row_off(step);
+        const int so = ro < 0 || nc == 0 ? 0 : ro;  // within the resource, also an empty one
         if constexpr (VEC) {
-            const int o = ro < 0 ? kOff : vo;
+            const unsigned o = ro < 0 ? kOff : vo;
 #pragma unroll
             for (int q = 0; q < NV; q++) {
                 const V w = __builtin_bit_cast(
-                    V, __builtin_amdgcn_raw_buffer_load_b128(rc, o + q * 16, ro < 0 ? 0 : ro, 0));
+                    V, __builtin_amdgcn_raw_buffer_load_b128(rc, o + q * 16, so, 0));
 #pragma unroll
                 for (int e = 0; e < VW; e++) v[q * VW + e] = w[e];
             }
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int o = ro < 0 || xl + e >= nx ? kOff : vo + e * SZ;
+                const unsigned o = ro < 0 || xl + e >= nx ? kOff : vo + e * SZ;
                 if constexpr (SZ == 4)
-                    v[e] = __builtin_bit_cast(
-                        T, __builtin_amdgcn_raw_buffer_load_b32(rc, o, ro < 0 ? 0 : ro, 0));
+                    v[e] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rc, o, so, 0));
                 else
-                    v[e] = __builtin_bit_cast(
-                        T, __builtin_amdgcn_raw_buffer_load_b64(rc, o, ro < 0 ? 0 : ro, 0));
+                    v[e] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rc, o, so, 0));
             }
         }
     };
@@ -754,7 +755,7 @@ __device__ __forceinline__ void nlb_chain_brick(
     auto store4 = [&](int step, const T (&v)[4]) {
         const int ro = row_off(step);
         if constexpr (VEC) {
-            const unsigned o = ro < 0 ? (unsigned)kOff : (unsigned)vo + (unsigned)ro;
+            const unsigned o = ro < 0 ? kOff : vo + (unsigned)ro;
 #pragma unroll
             for (int q = 0; q < NV; q++) {
                 V w;
@@ -766,7 +767,7 @@ __device__ __forceinline__ void nlb_chain_brick(
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const unsigned o =
-                    ro < 0 || xl + e >= nx ? (unsigned)kOff : (unsigned)vo + (unsigned)ro + e * SZ;
+                    ro < 0 || xl + e >= nx ? kOff : vo + (unsigned)ro + e * SZ;
                 if constexpr (SZ == 4)
                     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v[e]), rc, o, 0, 0);
                 else
