@@ -1130,8 +1130,8 @@ bool nlb_lds_kernels()
 }
 
 // What a launch over the bricks is part of: a projection or an apply by itself,
-// or a filter, whose applies also form the next projection.
-enum class NlbPass { Project, Apply, Filter };
+// a filter, whose applies also form the next projection, or the force integrals.
+enum class NlbPass { Project, Apply, Filter, Integrals };
 
 // Whether nlb_chain takes the launch: its register tiles hold every brick's
 // rows, 16 columns stay below 2^31 bytes, and its 128-column blocks have enough
@@ -1146,11 +1146,15 @@ enum class NlbPass { Project, Apply, Filter };
 // 382 -> 351, x 144 641 -> 638.  Apply: FP32 x 64 183 -> 188, x 72 272 -> 192, x
 // 144 385 -> 428, x 192 447 -> 456, x 200 551 -> 455; FP64 x 96 452 -> 495, x 128
 // 600 -> 540, x 192 857 -> 1012, x 200 955 -> 1030, x 256 1187 -> 1057.
-// SPARC_AMD_NLB=chain takes every width.
+// SPARC_AMD_NLB=chain takes every width.  The integrals, whose result is the sum
+// itself, stay with nlb_project_rs: it adds a brick's points in four chains of
+// 128, nlb_chain in one of 512 (rms error of FP32 integrals over 64^3 against 64
+// bits 5.4e-8 of the largest and 8.7e-8; in the filter the apply's own rounding
+// hides it, 2.7e-8 either way after 20 degrees).
 template <typename T>
 bool nlb_chain_takes(const sgpu_context *ctx, long ldo, int ncol, NlbPass pass)
 {
-    if (nlb_lds_kernels() || ctx->nl.max_np > 16 * Chain<T>::RTM ||
+    if (pass == NlbPass::Integrals || nlb_lds_kernels() || ctx->nl.max_np > 16 * Chain<T>::RTM ||
         16 * ldo * (long)sizeof(T) >= 0x7ffffff0L)
         return false;
     if (ctx->nlb_any_width) return true;
@@ -1696,7 +1700,7 @@ int project_alpha(sgpu_context *ctx, int ncol, const T *x, long ldx, double scal
         SGPU_CHECK(launch_nlb_project<T>(ctx, ncol, x, ldx,
                                          sizeof(T) == 8 ? (const T *)nl.phi64 : (const T *)nl.phi32,
                                          sizeof(T) == 8 ? (const T *)nl.phic64 : (const T *)nl.phic32,
-                                         part, NlbPass::Project));
+                                         part, NlbPass::Integrals));
         SGPU_HIP(hipGetLastError());
         const long total = (long)nl.n_alpha * ncol;
         nlb_reduce<T><<<(unsigned)((total + 255) / 256), 256, 0, ctx->stream>>>(

@@ -44,6 +44,21 @@ def test_nonlocal_integrals_match_oracle(gpu, monkeypatch, mode, dtype):
         assert rel_err(got[k], ref[k]) < (1e-12 if dtype == 0 else 2e-5), k
 
 
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_nonlocal_integrals_any_width(gpu, monkeypatch, dtype):
+    """Each column's integrals are the same sums whatever the width of its
+    block (the brick layout's wide projection adds in longer chains)."""
+    monkeypatch.setenv("SPARC_AMD_NL_MODE", "brick")
+    g, veff, nl, rng = small_case(n=(24, 20, 17), n_sites=5, rc=3.0, seed=32, lmax=1)
+    X = rng.uniform(-0.5, 0.5, (g.nd, 130))
+    with gpu.Context(g) as ctx:
+        ctx.set_nonlocal(nl)
+        wide = ctx.nonlocal_integrals(ctx.block(130, dtype).upload(X))
+        narrow = [ctx.nonlocal_integrals(ctx.block(c.shape[1], dtype).upload(c)) for c in np.split(X, [60], axis=1)
+                  for c in np.split(c, [50], axis=1)]
+    assert np.array_equal(wide, np.concatenate(narrow, axis=2))
+
+
 def test_nonlocal_integrals_psp_sic(gpu):
     """Real psp8 projectors (18 / 8 per atom, images across the faces)."""
     from oracle.forces import integrals
