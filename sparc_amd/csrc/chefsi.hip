@@ -1107,8 +1107,8 @@ __device__ __forceinline__ void wave_sum_f64(double (&d)[CW])
 // a row's two factors are read from their lanes.  A step then has one barrier:
 // the update also forms p = A22 v of the next step (its v follows from row
 // i + 1 alone), and p and the next row go to all waves through LDS.  n = 160:
-// 370 us, against 951 us for 1,024 threads with the packed triangle in LDS and
-// seven barriers a step.  Eight waves: with sixteen the vectors formed by
+// 370 us, n = 64: 75 us, against 951 and 199 us for 1,024 threads with the packed
+// triangle in LDS and seven barriers a step.  Eight waves: with sixteen the vectors formed by
 // every wave would take twice the issue slots, with four the rows would not
 // fit in the registers.
 constexpr int kTridMaxN = 180;   // three columns a lane (144 registers of matrix)
@@ -1159,7 +1159,10 @@ __global__ __launch_bounds__(64 * kTridWaves) void sytd2_lower_regs(double *__re
 #pragma unroll
             for (int q = 0; q < NQ; q++) {
                 const int c = ln + 64 * q;
-                if (c >= i && c < n) A[i * lda + c] = c == i ? dcur : c == i + 1 ? beta : v[q];
+                // values: as a choice of lvalues it kept every captured variable in
+                // scratch for one column a lane (n = 64: 168 us)
+                const double d = dcur, b = beta, u = v[q];
+                if (c >= i && c < n) A[i * lda + c] = c == i ? d : c == i + 1 ? b : u;
             }
             if (ln == 0) {
                 D[i] = dcur;
