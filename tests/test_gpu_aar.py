@@ -76,3 +76,29 @@ def test_aar_histories(gpu, oracle_mod, n, m, p, c):
     assert rel_err(x, xo) < 1e-6
     r = rhs + o.lap_vec_mult(x, c)[:, 0]
     assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(rhs) + 1e-13 * np.linalg.norm(x) * 60.0
+
+
+@pytest.mark.parametrize("n,bc,m,p", [((21, 21, 21), (0, 0, 0), 7, 6), ((21, 23, 26), (0, 0, 1), 5, 4),
+                                      ((24, 20, 31), (1, 0, 0), 7, 6), ((23, 26, 20), (0, 1, 0), 7, 3)])
+def test_aar_marching_step(gpu, oracle_mod, monkeypatch, n, bc, m, p):
+    """The one-launch step in its marching form (the default above 3.6 MB, here
+    forced): rows that end in a partly filled group, whole ones, and walls along
+    each axis, against the oracle.  Tolerances as in test_aar_histories."""
+    from sparc_amd.workloads import Grid
+    monkeypatch.setenv("SPARC_AMD_STENCIL_TILE", "20")
+    g = Grid(*n, 0.4, 0.42, 0.38, *bc)
+    rhs = np.random.default_rng(sum(n)).standard_normal(g.nd)
+    if not any(bc):
+        rhs -= rhs.mean()
+    o = oracle_mod.Oracle(g)
+    xo, it_o, rr_o = o.aar(np.zeros(g.nd), rhs, m=m, p=p, tol=1e-10, max_iter=3000)
+    with gpu.Context(g) as ctx:
+        x, it, rr, conv = ctx.AAR(np.zeros(g.nd), rhs, m=m, p=p, tol=1e-10, max_iter=3000)
+        assert ctx.stencil_kernel(gpu.F64, 1).startswith("stencil_march<")
+    assert conv and rr <= 1e-10
+    assert abs(it - it_o) <= max(12, it_o // 5)
+    if not any(bc):
+        x, xo = x - x.mean(), xo - xo.mean()
+    assert rel_err(x, xo) < 1e-6
+    r = rhs + o.lap_vec_mult(x, 0.0)[:, 0]
+    assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(rhs) + 1e-13 * np.linalg.norm(x) * 60.0

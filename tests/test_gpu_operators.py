@@ -138,6 +138,9 @@ def test_stencil_ring_fp32(gpu, oracle_mod, monkeypatch, cfg, n, bc, ncol):
     ((33, 6, 40), (0, 0, 0), 1),     # fewer rows than a tile's halo, z-chunks
     ((128, 13, 16), (1, 1, 1), 2),   # longest FP64 row
     ((256, 14, 16), (0, 0, 0), 1),   # longest FP32 row (FP64 takes the tiles)
+    ((77, 74, 40), (0, 0, 1), 1),    # 3.6 MB from 16 bytes a point on: near in both precisions,
+    ((77, 74, 40), (0, 1, 0), 3),    # marching in FP64 only,
+    ((77, 74, 40), (1, 0, 0), 4),    # and in both
 ])
 def test_stencil_vector_forms(gpu, oracle_mod, monkeypatch, form, n, bc, ncol):
     """The 16-bytes-per-thread stencils (20: marching, 21: for small blocks)
@@ -161,8 +164,13 @@ def test_stencil_vector_forms(gpu, oracle_mod, monkeypatch, form, n, bc, ncol):
             ctx.chebyshev_filter_dev(bx, by, 3, 2.0, 90.0, -3.0)
             y, prev = by.download(), bx.download()
             name = ctx.stencil_kernel(dt, ncol)
-        if n[0] <= (128 if dt == gpu.F64 else 256):
-            assert name.startswith({20: "stencil_march<", 21: "stencil_near<", None: "stencil_"}[form]), name
+        want = form
+        if form is None:  # near up to 3.6 MB
+            want = 21 if g.nd * ncol * (8 if dt == gpu.F64 else 4) <= 3600000 else 20
+        if want == 21 or n[0] <= (128 if dt == gpu.F64 else 256):
+            assert name.startswith({20: "stencil_march<", 21: "stencil_near<"}[want]), name
+        else:
+            assert name.startswith("stencil_tiled<"), name
         assert rel_err(y, yo) < tol and rel_err(prev, po) < tol
 
 
