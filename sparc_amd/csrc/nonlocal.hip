@@ -108,8 +108,7 @@ __device__ __forceinline__ long brick_point(int q, int x0, int y0, int z0, int n
 // consecutive points 4 lk .. 4 lk + 3 of its column li (one 16-byte access in
 // FP32, two in FP64) and the 16 lanes of a group read 16 columns' segments of
 // the row; the A operands (Phi_b rows of the same points) follow the same
-// assignment, which is also the one nlb_apply_rs's fused projection uses, so
-// both give the same bits.  NC columns per block share every Phi load (NC/16
+// assignment.  NC columns per block share every Phi load (NC/16
 // MFMAs per load); the next step's loads are issued before the current
 // step's MFMAs.  The four waves split the 512 points and their partial tiles
 // are summed in a fixed order (3 -> 2 -> 1 -> 0).  VEC: 16-byte loads (nx a
@@ -1549,7 +1548,8 @@ int build_sphere_layout(sgpu_context *ctx, int n_influence, const int *ndc, cons
             }
         coff += (long)qpad * npad;
     }
-    // an atom's images in the order they were given, whatever the entries' order
+    // an atom's images (and so the order of their sum) by colour, then in the order
+    // they were given, whatever the entries' places
     for (auto &v : imgs)
         std::sort(v.begin(), v.end(), [&](int x, int y) {
             return color[order[x]] != color[order[y]] ? color[order[x]] < color[order[y]]

@@ -132,9 +132,10 @@ struct sgpu_context {
     // on grids of 81-96 / 65-80 points), 13 / 14 = the same shapes as
     // stencil_rows when nx is exactly 96 / 80 (FP32); -1 (default) = the
     // fastest of 0 / 7 / 8 (9 / 10 below 16 columns, 11-14 where they fit),
-    // timed once per (precision, column count) and kept in tile_choice.  Above
-    // them, from 16 planes and 20 points along x: 20 = stencil_march, 21 =
-    // stencil_near, chosen by the block's bytes without timing.
+    // timed once per (precision, column count) and kept in tile_choice.  Before
+    // them, from 16 planes and 20 points along x: 21 = stencil_near for blocks of
+    // up to 3.6 MB, else 20 = stencil_march for rows of up to 128 points (FP64) /
+    // 256 (FP32), without timing.
     // SPARC_AMD_STENCIL_TILE fixes one at creation.
     int stencil_cfg = -1;
     std::map<std::pair<int, int>, int> tile_choice;
@@ -149,9 +150,10 @@ struct sgpu_context {
     // nlb_chain for any number of columns (SPARC_AMD_NLB=chain; by default
     // narrow blocks take the launches whose waves share their columns)
     bool nlb_any_width = false;
-    // eigensolves of up to 180 states reduce to tridiagonal form in one
-    // workgroup's LDS instead of rocsolver's dsytrd (SPARC_AMD_LDS_TRIDIAG=0
-    // keeps dsyevd everywhere)
+    // eigensolves of up to 180 states, and the last 180 columns of larger ones,
+    // reduce to tridiagonal form in one workgroup's registers instead of
+    // rocsolver's dsytrd (SPARC_AMD_LDS_TRIDIAG=0: the cooperative launch below
+    // for all columns)
     bool lds_tridiag = true;
     // larger eigensolves reduce to tridiagonal form in one cooperative launch
     // of this many workgroups, each holding a share of the rows in LDS

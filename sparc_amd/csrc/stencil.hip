@@ -982,7 +982,10 @@ void launch_ring(sgpu_context *ctx, const StencilParams<T> &p, int ncol)
 // 256, 512 or 1,024 threads hold, evened out over the tiles; the z-chunks are
 // those with the least rounds x (planes + 8), the 12 planes that every chunk
 // re-reads costing about 8 (measured: 52^3 x 160 FP32 71 us with one chunk, 61
-// with two, 70 with three; 78^3 x 480 FP32 677 / 652 / 748).
+// with two, 70 with three; 78^3 x 480 FP32 677 / 652 / 748).  Rows of more than
+// 64 groups (128 points in FP64, 256 in FP32) are left to the tiles: with the 12
+// rows that a block needs for its halo, those of more than 78 (80) groups pass
+// the 64 KB of LDS allowed here; the ones between are not measured.
 template <typename T>
 sgpu_march_plan plan_march(const sgpu_context *ctx, int ncol)
 {
@@ -1070,8 +1073,10 @@ void launch_march(sgpu_context *ctx, const StencilParams<T> &p, int ncol, const 
 constexpr long kNearBytes = 3600000;
 
 // Launches stencil_near or stencil_march where they apply (false: the tiles
-// below).  Grids of fewer than 16 planes, which no SCF or Poisson grid has,
-// keep the tuned tiles, whose bits do not depend on the tile.
+// below).  Grids of fewer than 16 planes are left to the tiles by default, only
+// to keep their results' bits: the vector forms are the faster ones there too
+// (40 x 40 x 15 x 24 FP64 24.6 -> 9.8 us, 64 x 64 x 8 x 200 FP32 32.6 -> 23.5,
+// 128 x 128 x 12 x 200 FP64 278 -> 259).
 template <typename T>
 bool launch_vec(sgpu_context *ctx, const StencilParams<T> &p, int ncol, int cfg)
 {
